@@ -13,10 +13,15 @@
 // sc*isum*bd for Q6_K (src/quant.c:422-434), isum*d*bd for Q8_0
 // (src/quant.c:279-285) -- and adds it to the (row, pair) accumulator in
 // unit order, so every output equals the reference's sequential fused dot.
+// Two fused multiply-adds stand for four of its operations where both their
+// inner products are exact (term_of below): the T = 512 layer of the
+// Qwen3-30B-A3B shape 242.9 -> 228.3 us, with 48 M VALU instructions in the
+// gate/up product where it had 58 M, and 40 M in down where it had 47 M.
 //
-// MFMA lane layout (v_mfma_i32_16x16x32_i8, checked on the device): A is
-// lane -> row lane%16, elements 8*(lane/16)..+7 of the unit; B is lane -> pair
-// lane%16, the same elements; D is lane -> pair lane%16, rows 4*(lane/16)+i.
+// MFMA lane layout (v_mfma_i32_16x16x32_i8, checked on the device): A, the
+// pairs, is lane -> pair lane%16, elements 8*(lane/16)..+7 of the unit; B, the
+// weights, is lane -> row lane%16, the same elements; D is lane -> row lane%16,
+// pairs 4*(lane/16)+i, so a row's scale and min are one value per lane.
 // The 8 elements of a lane's A and B may be in any order as long as both use
 // it: K-quant nibbles pair with activations stored [x0 x2 x4 x6 | x1 x3 x5 x7]
 // (the order a nibble dword unpacks to), Q8_0 with natural order.
@@ -62,7 +67,10 @@ struct MF {
 
 // The bits of the float 1.5 * 2^23: adding an integer |S| < 2^22 to them
 // gives the bits of the float 1.5 * 2^23 + S.
-constexpr int kQ6Magic = 0x4B400000;
+constexpr int kMagic = 0x4B400000;
+// The largest |bsum| whose product with any min is exact: a min is a half times
+// 0..3, at most 3 * 2047 = 6141 units of its last place, and 6141 * 2732 < 2^24.
+constexpr float kBsumExact = 2732.0f;
 
 // Four bits (bits 0..3 of x) to bit 4 of 4 bytes.
 __device__ inline uint32_t bits4_to_b4(uint32_t x) { return spread4(x) << 4; }
@@ -383,8 +391,8 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
   float* mnl = reinterpret_cast<float*>(smem + G::O_M + wave * G::SCL);
 
   // The stage loop and the outputs, in two forms.  Full: an MFMA per (unit,
-  // matrix, 16-row tile, 16-pair column tile), A = weights, B = pairs; lane
-  // (ln, kg) accumulates rows 4 kg + i of pair 16 j + ln.  Skinny (a work
+  // matrix, 16-row tile, 16-pair tile), A = pairs, B = weights; lane (ln, kg)
+  // accumulates row ln of pairs 16 j + 4 kg + i.  Skinny (a work
   // item of at most 4 pairs): A = the pairs with each pair's 32 elements split
   // into 4 k-quarters on 4 A rows (row 4 t + q holds pair t's quarter q, zeros
   // elsewhere), B = weights; lane (ln, kg) receives the 4 quarter sums of pair
@@ -434,6 +442,7 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
       // scales and mins of the wave's (matrix, unit, row)s, entry
       // (m * 8 + s) * WR + rr: lane (m, rr, half) decodes row rr's header once
       // for units 4 half .. 4 half + 3
+      bool odd = false;  // a block scale that is not finite, or an inexact m * bsum
       for (int i = lane; i < NMAT * WR * 2; i += 64) {
         const int m = i / (2 * WR), rem = i - m * 2 * WR;
         const int rr = rem >> 1, half = rem & 1;
@@ -442,6 +451,8 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
         if (4 * half < su && row < a.rows) {
           const int hd = (int)(((uint32_t)row * (uint32_t)rb + s0) & 15u);
           unit_scales4<TYPE>(wl, (m * WR + rr) * G::SLOT + hd, 4 * half, su, sc, mn);
+#pragma unroll
+          for (int q = 0; q < 4; q++) odd |= !(__builtin_fabsf(sc[q] + mn[q]) < __builtin_inff());
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -463,19 +474,50 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
 #pragma unroll
           for (int r = 0; r < RA; r++) q6[m][r] = q6_ref((m * WR + 16 * r + ln) * G::SLOT + hA[r], kg);
       }
-      auto term_of = [&](float sc, float mn, int isum, float bd, float bsf, int bs) {
-        if constexpr (MF<TYPE>::kMin) return (sc * (float)isum - mn * bsf) * bd;
-        else if constexpr (TYPE == QR_T_Q6_K) return sc * (float)(isum - 32 * bs) * bd;
-        else return (float)isum * sc * bd;
+      // Whether this stage's terms may take the fused forms below: every block
+      // scale of the wave's rows finite (checked where they were decoded) and,
+      // with mins, |bsum| <= kBsumExact in every unit of the item's pairs.
+      if constexpr (MF<TYPE>::kMin) {
+#pragma unroll
+        for (int k = 0; k < G::NTOK * 8 / 64; k++) {
+          const int i = k * 64 + lane, tt = i >> 3;
+          const float bsf =
+              *reinterpret_cast<const float*>(as + tt * (16 * G::APC) + (i & 7) * kXQ + 36);
+          odd |= tt < np && __builtin_fabsf(bsf) > kBsumExact;
+        }
+      }
+      const bool fused = __builtin_amdgcn_ballot_w64(odd) == 0;  // wave-uniform
+      // One term from the accumulator bits of 1.5 * 2^23 + isum.  Fused: the
+      // first multiply-add is RN(sc * isum), as nsc = -sc * 1.5 * 2^23 is exact
+      // (sc has at most 19 significant bits); m * bsum is exact too, so the
+      // second is RN(RN(sc * isum) - RN(m * bsum)): the reference's bits in
+      // 4 operations (3 without mins) where the separate ones take 6 (4).
+      auto term_of = [&](auto fused_tag, float sc, float nsc, float mn, int bits, float bd,
+                         float bsf) {
+        if constexpr (decltype(fused_tag)::value) {
+          float t = __builtin_fmaf(sc, __builtin_bit_cast(float, bits), nsc);
+          if constexpr (MF<TYPE>::kMin) t = __builtin_fmaf(-mn, bsf, t);
+          return t * bd;
+        } else {
+          float t = sc * (float)(bits - kMagic);
+          if constexpr (MF<TYPE>::kMin) t = t - mn * bsf;
+          return t * bd;
+        }
       };
-      auto unit_step = [&](int s) {
+      auto unit_step = [&](int s, auto fused_tag) {
         long Wq[NMAT][RA];
+        float sc[NMAT][RA], nsc[NMAT][RA], mn[NMAT][RA];
 #pragma unroll
         for (int m = 0; m < NMAT; m++)
 #pragma unroll
-          for (int r = 0; r < RA; r++)
+          for (int r = 0; r < RA; r++) {
             if constexpr (TYPE == QR_T_Q6_K) Wq[m][r] = unit_a_q6(wl, q6[m][r], s);
             else Wq[m][r] = unit_a<TYPE>(wl, (m * WR + 16 * r + ln) * G::SLOT + hA[r], s, kg);
+            const int si = (m * 8 + s) * WR + 16 * r + ln;
+            sc[m][r] = scl[si];
+            mn[m][r] = mnl[si];
+            nsc[m][r] = sc[m][r] * -12582912.0f;  // -1.5 * 2^23
+          }
         if constexpr (SK) {
           // A: pair ln / 4's quarter ln % 4 on A row ln (zeros in the other
           // k-groups); the term's pair is kg
@@ -486,69 +528,66 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
           const uint8_t* rt = as + kg * (16 * G::APC) + s * kXQ;
           const float bd = *reinterpret_cast<const float*>(rt + 32);
           const float bsf = *reinterpret_cast<const float*>(rt + 36);
-          const int bs = *reinterpret_cast<const int*>(rt + 40);
+          const int bs = TYPE == QR_T_Q6_K ? *reinterpret_cast<const int*>(rt + 40) : 0;
 #pragma unroll
           for (int m = 0; m < NMAT; m++)
 #pragma unroll
             for (int r = 0; r < RA; r++) {
-              const v4i zero = {0, 0, 0, 0};
-              const v4i Dv = __builtin_amdgcn_mfma_i32_16x16x32_i8(Aq, Wq[m][r], zero, 0, 0, 0);
-              const int isum = (Dv[0] + Dv[1]) + (Dv[2] + Dv[3]);
-              const int si = (m * 8 + s) * WR + 16 * r + ln;
-              acc[m][r][0][0] += term_of(scl[si], mnl[si], isum, bd, bsf, bs);
+              const v4i c0 = {kMagic, 0, 0, 0};
+              const v4i Dv = __builtin_amdgcn_mfma_i32_16x16x32_i8(Aq, Wq[m][r], c0, 0, 0, 0);
+              const int bits = (Dv[0] + Dv[1]) + (Dv[2] + Dv[3]) - 32 * bs;
+              acc[m][r][0][0] += term_of(fused_tag, sc[m][r], nsc[m][r], mn[m][r], bits, bd, bsf);
             }
         } else {
 #pragma unroll
           for (int j = 0; j < NJA; j++) {
-            const uint8_t* rec = as + (16 * j + ln) * (16 * G::APC) + s * kXQ;
-            const uint2 bq = *reinterpret_cast<const uint2*>(rec + 8 * kg);
-            const long B = (long)((uint64_t)bq.x | ((uint64_t)bq.y << 32));
-            const float bd = *reinterpret_cast<const float*>(rec + 32);
-            const float bsf = *reinterpret_cast<const float*>(rec + 36);
-            const int bs = *reinterpret_cast<const int*>(rec + 40);
-            // Q6_K: the accumulator starts at the bits of 1.5 * 2^23, so each
-            // exact sum S (|S| <= 32 * 63 * 127 < 2^22) comes out as the bits
-            // of the float 1.5 * 2^23 + S; less 1.5 * 2^23 + 32 bs (exact
-            // too) that is (float)(S - 32 bs) in one exact subtraction, the
-            // value the reference's (float)isum holds
-            const float q6m = __builtin_bit_cast(float, kQ6Magic + 32 * bs);
+            const uint2 bq = *reinterpret_cast<const uint2*>(
+                as + (16 * j + ln) * (16 * G::APC) + s * kXQ + 8 * kg);
+            const long A = (long)((uint64_t)bq.x | ((uint64_t)bq.y << 32));
+            float2 bb[4];  // (bd, bsf) of the lane's four pairs
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+              bb[i] = *reinterpret_cast<const float2*>(
+                  as + (16 * j + 4 * kg + i) * (16 * G::APC) + s * kXQ + 32);
+            // the accumulators start at the bits of 1.5 * 2^23, so an exact sum
+            // S (|S| < 2^22) comes out as the bits of the float 1.5 * 2^23 + S;
+            // Q6_K's stored quants carry an offset of 32, which one more
+            // product against a constant -32 takes out for all the rows at once
+            v4i c0 = v4i{kMagic, kMagic, kMagic, kMagic};
+            if constexpr (TYPE == QR_T_Q6_K)
+              c0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, (long)0xE0E0E0E0E0E0E0E0ull, c0, 0, 0, 0);
 #pragma unroll
             for (int m = 0; m < NMAT; m++)
 #pragma unroll
               for (int r = 0; r < RA; r++) {
-                const v4i c0 = TYPE == QR_T_Q6_K ? v4i{kQ6Magic, kQ6Magic, kQ6Magic, kQ6Magic}
-                                                 : v4i{0, 0, 0, 0};
-                const v4i Dv = __builtin_amdgcn_mfma_i32_16x16x32_i8(Wq[m][r], B, c0, 0, 0, 0);
-                const int si = (m * 8 + s) * WR + 16 * r + 4 * kg;
-                const float4 sc4 = *reinterpret_cast<const float4*>(scl + si);
-                const float4 mn4 = *reinterpret_cast<const float4*>(mnl + si);
-                const float scv[4] = {sc4.x, sc4.y, sc4.z, sc4.w};
-                const float mnv[4] = {mn4.x, mn4.y, mn4.z, mn4.w};
+                const v4i Dv = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, Wq[m][r], c0, 0, 0, 0);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                  if constexpr (TYPE == QR_T_Q6_K) {
-                    // each element passes through an empty asm before its
-                    // float view: without it this compiler (ROCm 7.2 clang)
-                    // folds the four subtractions of the float views of an
-                    // MFMA result's elements into one, on element 0
-                    int di = Dv[i];
-                    asm("" : "+v"(di));
-                    acc[m][r][j][i] += scv[i] * (__builtin_bit_cast(float, di) - q6m) * bd;
-                  } else {
-                    acc[m][r][j][i] += term_of(scv[i], mnv[i], Dv[i], bd, bsf, bs);
-                  }
+                  // each element passes through an empty asm before its float
+                  // view: without it this compiler (ROCm 7.2 clang) folds the
+                  // operations on the float views of an MFMA result's elements
+                  // into one, on element 0
+                  int di = Dv[i];
+                  asm("" : "+v"(di));
+                  acc[m][r][j][i] += term_of(fused_tag, sc[m][r], nsc[m][r], mn[m][r], di, bb[i].x,
+                                             bb[i].y);
                 }
               }
           }
         }
       };
-      if (su == 8) {
-        // every stage of a K-quant, and whole Q8_0 stages: unrolled, so the
-        // units' LDS reads and MFMAs interleave
+      if (fused) {
+        if (su == 8) {
+          // every stage of a K-quant, and whole Q8_0 stages: unrolled, so the
+          // units' LDS reads and MFMAs interleave
 #pragma unroll
-        for (int s = 0; s < 8; s++) unit_step(s);
+          for (int s = 0; s < 8; s++) unit_step(s, std::true_type{});
+        } else {
+          for (int s = 0; s < su; s++) unit_step(s, std::true_type{});
+        }
       } else {
-        for (int s = 0; s < su; s++) unit_step(s);
+#pragma unroll 1
+        for (int s = 0; s < su; s++) unit_step(s, std::false_type{});
       }
     }
 
@@ -558,8 +597,8 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
         *tt = kg;
         *row = rw0 + 16 * r + ln;
       } else {
-        *tt = 16 * j + ln;
-        *row = rw0 + 16 * r + 4 * kg + i;
+        *tt = 16 * j + 4 * kg + i;
+        *row = rw0 + 16 * r + ln;
       }
     };
     constexpr int OJ = NJA, OI = SK ? 1 : 4;
