@@ -1158,7 +1158,6 @@ struct qr_decoder {
   float *pv = nullptr, *pao = nullptr, *patt = nullptr;
   int32_t* pst = nullptr;   // [cap][2]: token, position of every prompt position
   uint8_t* prec = nullptr;  // activation records [pcap][max(dim, q_dim) / 32]
-  int32_t *poff = nullptr, *pperm = nullptr, *ptiles = nullptr;
   uint8_t* pmoe = nullptr;
   const float* prec_src = nullptr;  // the rows prec holds records of (nullptr: none)
   int prec_perm = 0;
@@ -1385,26 +1384,6 @@ hipError_t enqueue_step(qr_decoder* d, float* logits, float* xout, hipStream_t s
   return hipSuccess;
 }
 
-// A single-"expert" dispatch of T rows for the grouped MFMA product:
-// offsets {0, T}, the identity permutation, tiles {0, ceil(T / tile)}; with
-// tiles2, also {0, ceil(T / 32)} there (a chunk's products take 16- or
-// 32-pair items by their row count).
-__global__ __launch_bounds__(256) void k_rows_dispatch(int T, int tile, int32_t* off,
-                                                       int32_t* perm, int32_t* tiles,
-                                                       int32_t* tiles2) {
-  for (int i = threadIdx.x; i < T; i += blockDim.x) perm[i] = i;
-  if (threadIdx.x == 0) {
-    off[0] = 0;
-    off[1] = T;
-    tiles[0] = 0;
-    tiles[1] = (T + tile - 1) / tile;
-    if (tiles2) {
-      tiles2[0] = 0;
-      tiles2[1] = (T + 31) / 32;
-    }
-  }
-}
-
 // y[t][.] = W x[t] for T rows of x (a prompt chunk), each row exactly as
 // matmul_q_dev computes it for one token: fp32 weights through the build's
 // order with all T rows at once; K-quant (row-major or tiled) and C99-order
@@ -1413,8 +1392,7 @@ __global__ __launch_bounds__(256) void k_rows_dispatch(int T, int tile, int32_t*
 // fused dot's; Q8_0 in a lane order and llama.cpp-layout K-quants through the
 // GEMV, four rows per launch.
 // The records of x are quantized unless `records` says the previous call
-// left those of the same x (and the same record order) in d->prec; the chunk's
-// single-expert dispatch lists are written once per chunk (prefill_rows_setup).
+// left those of the same x (and the same record order) in d->prec.
 // Pairs per work item of the T-row products: a dense matrix has one
 // "expert", so the items are what spreads it over the CUs.  16 for chunks
 // below 256 rows (128-token chunks: 71 ms for 512 prompt tokens against 75
@@ -1455,9 +1433,8 @@ hipError_t matmul_rows_dev(qr_decoder* d, const void* w, uint32_t type, const fl
     }
     const size_t slice = qr_wrow_bytes((int)base, dd) * (size_t)n;
     return expert_mfma_launch((int)base, false, static_cast<const uint8_t*>(w), nullptr, slice, 1,
-                              1, n, dd, d->prec, 1, d->poff, d->pperm,
-                              tile == 16 ? d->ptiles : d->ptiles + 2, y, n,
-                              (T + tile - 1) / tile + 1, tile, nullptr, false, s, tiled);
+                              1, n, dd, d->prec, 0, nullptr, nullptr, nullptr, nullptr, T, y, n,
+                              tile, nullptr, false, s, tiled);
   }
   for (int t0 = 0; t0 < T; t0 += 4) {
     const int nt = T - t0 < 4 ? T - t0 : 4;
@@ -1480,11 +1457,6 @@ hipError_t enqueue_prefill_chunk(qr_decoder* d, int T, const int32_t* st, int pe
                                  hipStream_t s) {
   hipError_t e;
   const int dim = d->dim;
-  // the chunk's single-expert dispatch of its T rows (in the items
-  // matmul_rows_dev launches)
-  hipLaunchKernelGGL(k_rows_dispatch, dim3(1), dim3(256), 0, s, T, 16, d->poff, d->pperm,
-                     d->ptiles, d->ptiles + 2);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
   d->prec_src = nullptr;
   hipLaunchKernelGGL(k_embed, dim3(T), dim3(256), 0, s, static_cast<const uint8_t*>(d->tok_embd),
                      (int)d->tok_type, d->tok_row, st, dim, d->px);
@@ -1631,15 +1603,6 @@ int check_layer_weights(const qr_model* m, int l, int order) {
 }
 
 }  // namespace
-
-namespace qr {
-hipError_t rows_dispatch_launch(int T, int tile, int32_t* off, int32_t* perm, int32_t* tiles,
-                                hipStream_t st) {
-  hipLaunchKernelGGL(k_rows_dispatch, dim3(1), dim3(256), 0, st, T, tile, off, perm, tiles,
-                     (int32_t*)nullptr);
-  return hipGetLastError();
-}
-}  // namespace qr
 
 extern "C" {
 
@@ -1999,9 +1962,7 @@ static int prefill_workspace(qr_decoder* d, int chunk) {
   const size_t o_att = o_ao + up(T * d->qd * 4);
   const size_t o_st = o_att + up(T * d->nh * (size_t)d->cap * 4);
   const size_t o_rec = o_st + up((size_t)d->cap * 8);
-  const size_t o_off = o_rec + up(T * (size_t)(wide / 32) * 48);
-  const size_t o_perm = o_off + 256, o_tiles = o_perm + up(T * 4);
-  const size_t o_moe = o_tiles + 256, total = o_moe + up(moe_bytes);
+  const size_t o_moe = o_rec + up(T * (size_t)(wide / 32) * 48), total = o_moe + up(moe_bytes);
   void* p = nullptr;
   const hipError_t e = hipMalloc(&p, total);
   if (e != hipSuccess)
@@ -2020,9 +1981,6 @@ static int prefill_workspace(qr_decoder* d, int chunk) {
   d->patt = reinterpret_cast<float*>(b + o_att);
   d->pst = reinterpret_cast<int32_t*>(b + o_st);
   d->prec = b + o_rec;
-  d->poff = reinterpret_cast<int32_t*>(b + o_off);
-  d->pperm = reinterpret_cast<int32_t*>(b + o_perm);
-  d->ptiles = reinterpret_cast<int32_t*>(b + o_tiles);
   d->pmoe = b + o_moe;
   return QR_OK;
 }

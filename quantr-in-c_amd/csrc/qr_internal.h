@@ -103,9 +103,6 @@ struct MoeScratch {
   float* ush;         // [T][sh_hidden]  its up rows (GEMV path)
   uint8_t* xqs;       // [T][dim/32]     records of xb in its up type's order (MFMA path)
   uint8_t* hqs;       // [T][sh_hidden/32] records of its hb (MFMA path)
-  int32_t* shoff;     // [2]   single-"expert" dispatch of the T tokens
-  int32_t* shtiles;   // [2]
-  int32_t* shperm;    // [T]
   float* hu;          // [T*K][hidden]  up rows of llama.cpp-layout experts (else null)
 };
 size_t moe_scratch_bytes(const qr_moe_layer* L, int T);
@@ -115,7 +112,7 @@ hipError_t moe_route_launch(const qr_moe_layer* L, const float* xb, int T, int o
                             hipStream_t st);
 hipError_t moe_dispatch_launch(const int32_t* idx, int T, int K, int E, int tile, int32_t* counts,
                                int32_t* offsets, int32_t* tiles, int32_t* perm, int32_t* inv,
-                               hipStream_t st);
+                               hipStream_t st, int4* table = nullptr);
 // path: QR_MOE_PATH_* (include/qr_hip.h); AUTO picks by the pairs per expert.
 // norm_w (one token, where moe_t1_norm_ok): xb is written, not read -- the
 // router's launch forms xb = rmsnorm_ref(x, norm_w) (src/kernels.c:170-180)
@@ -126,10 +123,6 @@ hipError_t moe_forward_launch(const qr_moe_layer* L, float* x, const float* xb, 
                               const MoeScratch& s, hipStream_t st, int path = QR_MOE_PATH_AUTO,
                               const float* norm_w = nullptr);
 hipError_t softmax_launch(float* x, int rows, int n, hipStream_t st);
-// qr_decode.hip: a single-"expert" dispatch of T rows for the grouped MFMA
-// product (offsets {0, T}, the identity permutation, tiles {0, ceil(T / tile)}).
-hipError_t rows_dispatch_launch(int T, int tile, int32_t* off, int32_t* perm, int32_t* tiles,
-                                hipStream_t st);
 
 // qr_moe_t1.hip
 bool router1_ok(int dim);
@@ -170,10 +163,14 @@ hipError_t quant_rows_launch(const float* x, int xstride, int nrows, int cols, b
 // Pairs per work item of the grouped MFMA products for T tokens (the
 // dispatch's tile size).
 int mfma_tile(int T, int K, int E);
+// P (token, slot) pairs.  offsets null: one matrix (E = 1) and P rows in order
+// (perm and tiles unread).  table (optional, P entries): the dispatch's work
+// items as (expert, first position, pairs).
 hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const uint8_t* W2,
                               size_t slice, int E, int K, int rows, int cols, const uint8_t* XQ,
                               int x_by_token, const int32_t* offsets, const int32_t* perm,
-                              const int32_t* tiles, float* Y, int ystride, int items, int tile,
-                              uint8_t* QO, bool qperm, hipStream_t st, bool tiled = false);
+                              const int32_t* tiles, const int4* table, int P, float* Y,
+                              int ystride, int tile, uint8_t* QO, bool qperm, hipStream_t st,
+                              bool tiled = false);
 
 }  // namespace qr

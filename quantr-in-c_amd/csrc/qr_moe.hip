@@ -62,7 +62,8 @@ size_t moe_scratch_bytes(const qr_moe_layer* L, int T) {
     b += a256((size_t)T * sh * 4);                  // ush
     b += a256((size_t)T * (L->dim / 32) * 48);      // xqs
     b += a256((size_t)T * (sh / 32) * 48);          // hqs
-    b += a256(2 * 4) * 2 + a256((size_t)T * 4);     // shoff, shtiles, shperm
+    b += a256(2 * 4) * 2 + a256((size_t)T * 4);     // unused; counted, so that a fixed
+                                                    // scratch takes the same layers as ever
   }
   if (L->up_type & QR_GGML) b += a256(P * (size_t)L->hidden * 4);  // hu
   return b;
@@ -94,14 +95,10 @@ void moe_scratch_carve(void* base, const qr_moe_layer* L, int T, MoeScratch* s) 
   s->hq = take(P * (size_t)(L->hidden / 32) * 48);
   s->ush = nullptr;
   s->xqs = s->hqs = nullptr;
-  s->shoff = s->shtiles = s->shperm = nullptr;
   if (sh) {
     s->ush = reinterpret_cast<float*>(take((size_t)T * sh * 4));
     s->xqs = take((size_t)T * (L->dim / 32) * 48);
     s->hqs = take((size_t)T * (sh / 32) * 48);
-    s->shoff = reinterpret_cast<int32_t*>(take(2 * 4));
-    s->shtiles = reinterpret_cast<int32_t*>(take(2 * 4));
-    s->shperm = reinterpret_cast<int32_t*>(take((size_t)T * 4));
   }
   s->hu = nullptr;
   if (L->up_type & QR_GGML) s->hu = reinterpret_cast<float*>(take(P * (size_t)L->hidden * 4));
@@ -183,24 +180,30 @@ hipError_t softmax_launch(float* x, int rows, int n, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// Dispatch: one workgroup of kDispThreads threads (qr_tokens.h).
+// Dispatch: one workgroup of kDispThreads threads (qr_tokens.h).  k_iota: the
+// positions of pairs that were not dispatched (pair p at p).
 // ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_iota(int32_t* __restrict__ inv, int P) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p < P) inv[p] = p;
+}
 __global__ __launch_bounds__(kDispThreads) void k_dispatch(const int32_t* __restrict__ idx, int P,
                                                            int E, int tile,
                                                            int32_t* __restrict__ counts,
                                                            int32_t* __restrict__ offsets,
                                                            int32_t* __restrict__ tiles,
                                                            int32_t* __restrict__ perm,
-                                                           int32_t* __restrict__ inv) {
-  dispatch_wg(idx, P, E, tile, counts, offsets, tiles, perm, inv);
+                                                           int32_t* __restrict__ inv,
+                                                           int4* __restrict__ table) {
+  dispatch_wg(idx, P, E, tile, counts, offsets, tiles, perm, inv, table);
 }
 
 hipError_t moe_dispatch_launch(const int32_t* idx, int T, int K, int E, int tile, int32_t* counts,
                                int32_t* offsets, int32_t* tiles, int32_t* perm, int32_t* inv,
-                               hipStream_t st) {
+                               hipStream_t st, int4* table) {
   if (E > 256) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_dispatch, dim3(1), dim3(kDispThreads), 0, st, idx, T * K, E, tile, counts,
-                     offsets, tiles, perm, inv);
+                     offsets, tiles, perm, inv, table);
   return hipGetLastError();
 }
 
@@ -698,20 +701,17 @@ static hipError_t shared_expert(const qr_moe_layer* L, const float* xb, int T, c
   } else if (T > 4 && same_up && aligned && mfma_type_ok(ut) && mfma_type_ok(dt) &&
              dim % qr_block_elems(ut) == 0 && sh % 32 == 0 && sh % qr_block_elems(dt) == 0) {
     const int tile = mfma_tile(T, 1, 1);
-    const int items = (T + tile - 1) / tile + 1;
-    if ((e = rows_dispatch_launch(T, tile, s.shoff, s.shperm, s.shtiles, st)) != hipSuccess)
-      return e;
     if ((e = quant_rows_launch(xb, dim, T, dim, ut != QR_T_Q8_0, s.xqs, st)) != hipSuccess) return e;
     const size_t su = qr_wrow_bytes(ut, dim) * (size_t)sh;
     const size_t sd = qr_wrow_bytes(dt, sh) * (size_t)dim;
     e = expert_mfma_launch(ut, true, static_cast<const uint8_t*>(L->sh_up),
                            static_cast<const uint8_t*>(L->sh_gate), su, 1, 1, sh, dim, s.xqs, 0,
-                           s.shoff, s.shperm, s.shtiles, s.hbs, sh, items, tile, s.hqs,
+                           nullptr, nullptr, nullptr, nullptr, T, s.hbs, sh, tile, s.hqs,
                            dt != QR_T_Q8_0, st);
     if (e != hipSuccess) return e;
     e = expert_mfma_launch(dt, false, static_cast<const uint8_t*>(L->sh_down), nullptr, sd, 1, 1,
-                           dim, sh, s.hqs, 0, s.shoff, s.shperm, s.shtiles, s.ysh, dim, items, tile,
-                           nullptr, false, st);
+                           dim, sh, s.hqs, 0, nullptr, nullptr, nullptr, nullptr, T, s.ysh, dim,
+                           tile, nullptr, false, st);
     if (e != hipSuccess) return e;
   } else {
     const int nt = T >= 8 ? 8 : T >= 4 ? 4 : T >= 2 ? 2 : 1;
@@ -777,7 +777,8 @@ static hipError_t moe_forward_ggml(const qr_moe_layer* L, float* x, const float*
   e = gemv_ggml_pairs_launch(dt, L->down, sd, s.idx, E, 1, s.hb, L->hidden, s.y, L->dim, L->dim,
                              L->hidden, P, st);
   if (e != hipSuccess) return e;
-  if ((e = rows_dispatch_launch(P, 1, s.offsets, s.inv, s.tiles, st)) != hipSuccess) return e;
+  hipLaunchKernelGGL(k_iota, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, st, s.inv, P);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
   return combine_launch(x, s.y, s.inv, s.wts, T, K, L->dim, nullptr, nullptr, st);
 }
 
@@ -866,18 +867,21 @@ hipError_t moe_forward_launch(const qr_moe_layer* L, float* x, const float* xb, 
     if (e != hipSuccess) return e;
     e = route_rank_launch(s.logits, T, E, K, nullptr, s.idx, s.wts, xb, L->dim, perm_x, s.xq, st);
     if (e != hipSuccess) return e;
+    // the work items' table (at most P of them) in the hidden rows' place:
+    // gate/up writes records here, not rows
+    int4* table = reinterpret_cast<int4*>(s.hb);
+    static_assert(sizeof(int4) <= 32 * sizeof(float), "a pair's hidden row holds its item");
     e = moe_dispatch_launch(s.idx, T, K, E, kTile, s.counts, s.offsets, s.tiles, s.perm, s.inv,
-                            st);
+                            st, table);
     if (e != hipSuccess) return e;
-    const int items = (P + kTile - 1) / kTile + E;  // >= sum_e ceil(count_e / kTile)
     e = expert_mfma_launch((int)L->up_type, true, static_cast<const uint8_t*>(L->up),
                            static_cast<const uint8_t*>(L->gate), su, E, K, L->hidden, L->dim, s.xq,
-                           1, s.offsets, s.perm, s.tiles, s.hb, L->hidden, items, kTile, s.hq,
+                           1, s.offsets, s.perm, s.tiles, table, P, nullptr, L->hidden, kTile, s.hq,
                            L->down_type != QR_T_Q8_0, st);
     if (e != hipSuccess) return e;
     e = expert_mfma_launch((int)L->down_type, false, static_cast<const uint8_t*>(L->down), nullptr,
-                           sd, E, K, L->dim, L->hidden, s.hq, 0, s.offsets, s.perm, s.tiles, s.y,
-                           L->dim, items, kTile, nullptr, false, st);
+                           sd, E, K, L->dim, L->hidden, s.hq, 0, s.offsets, s.perm, s.tiles, table,
+                           P, s.y, L->dim, kTile, nullptr, false, st);
     if (e != hipSuccess) return e;
     if (sh) {
       e = shared_expert(L, xb, T, s, st, sg);
@@ -937,19 +941,18 @@ hipError_t moe_forward_launch(const qr_moe_layer* L, float* x, const float* xb, 
     const int kTile = mfma_tile(T, K, E);  // pairs per MFMA work item
     e = moe_dispatch_launch(s.idx, T, K, E, kTile, s.counts, s.offsets, s.tiles, s.perm, s.inv, st);
     if (e != hipSuccess) return e;
-    const int items = (P + kTile - 1) / kTile + E;  // >= sum_e ceil(count_e / kTile)
     e = quant_rows_launch(xb, L->dim, T, L->dim, L->up_type != QR_T_Q8_0, s.xq, st);
     if (e != hipSuccess) return e;
     e = expert_mfma_launch((int)L->up_type, true, static_cast<const uint8_t*>(L->up),
                            static_cast<const uint8_t*>(L->gate), su, E, K, L->hidden, L->dim, s.xq,
-                           1, s.offsets, s.perm, s.tiles, s.hb, L->hidden, items, kTile, nullptr,
-                           false, st);
+                           1, s.offsets, s.perm, s.tiles, nullptr, P, s.hb, L->hidden, kTile,
+                           nullptr, false, st);
     if (e != hipSuccess) return e;
     e = quant_rows_launch(s.hb, L->hidden, P, L->hidden, L->down_type != QR_T_Q8_0, s.hq, st);
     if (e != hipSuccess) return e;
     e = expert_mfma_launch((int)L->down_type, false, static_cast<const uint8_t*>(L->down), nullptr,
-                           sd, E, K, L->dim, L->hidden, s.hq, 0, s.offsets, s.perm, s.tiles, s.y,
-                           L->dim, items, kTile, nullptr, false, st);
+                           sd, E, K, L->dim, L->hidden, s.hq, 0, s.offsets, s.perm, s.tiles, nullptr,
+                           P, s.y, L->dim, kTile, nullptr, false, st);
     if (e != hipSuccess) return e;
   } else {
   const int nt = pick_tile(P, E);

@@ -75,25 +75,42 @@ constexpr float kBsumExact = 2732.0f;
 // Four bits (bits 0..3 of x) to bit 4 of 4 bytes.
 __device__ inline uint32_t bits4_to_b4(uint32_t x) { return spread4(x) << 4; }
 
-// A operand of unit s of a staged row (`o` = byte offset of the row's stage
-// in the LDS slot area `wl`): the lane's 8 elements (k-group kg) as 8 int8.
+// LDS reads at a byte address held in a register plus a constant: the offset
+// then sits in the instruction.  lds_base keeps the compiler from folding the
+// address back into its parts, which it would add up again for every read that
+// it pairs.
+__device__ inline uint32_t lds_base(const void* p) {
+  uint32_t a = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)p;
+  asm("" : "+v"(a));
+  return a;
+}
+template <typename T>
+__device__ inline T lds_at(uint32_t base, int off) {
+  return *(const __attribute__((address_space(3))) T*)(uintptr_t)(base + (uint32_t)off);
+}
+
+// A lane's 8 int8 elements (k-group kg) of unit s of a staged row: the row's
+// stage starts at LDS byte address `row`, `rowk` = row + 4 kg.
 template <int TYPE>
-__device__ inline long unit_a(const uint32_t* wl, int o, int s, int kg) {
+__device__ inline long unit_w(uint32_t row, uint32_t rowk, int s, int kg) {
   uint32_t lo, hi;
   if constexpr (TYPE == QR_T_Q4_K) {
-    const uint32_t w = wl[(o + 16 + 16 * s + 4 * kg) >> 2];  // aligned
+    const uint32_t w = lds_at<uint32_t>(rowk, 16 + 16 * s);  // aligned
     lo = w & 0x0F0F0F0Fu;
     hi = (w >> 4) & 0x0F0F0F0Fu;
   } else if constexpr (TYPE == QR_T_Q5_K) {
-    const uint32_t w = wl[(o + 48 + 16 * s + 4 * kg) >> 2];
-    const uint32_t t = (wl[(o + 16 + 4 * s) >> 2] >> (8 * kg)) & 0xFFu;
+    const uint32_t w = lds_at<uint32_t>(rowk, 48 + 16 * s);
+    const uint32_t t = (lds_at<uint32_t>(row, 16 + 4 * s) >> (8 * kg)) & 0xFFu;
     const uint32_t ev = (t & 1u) | ((t >> 1) & 2u) | ((t >> 2) & 4u) | ((t >> 3) & 8u);
     const uint32_t od = ((t >> 1) & 1u) | ((t >> 2) & 2u) | ((t >> 3) & 4u) | ((t >> 4) & 8u);
     lo = (w & 0x0F0F0F0Fu) | bits4_to_b4(ev);
     hi = ((w >> 4) & 0x0F0F0F0Fu) | bits4_to_b4(od);
-  } else {  // Q8_0 (Q6_K: unit_a_q6): block s, bytes 2 + 8 kg .. +7
-    lo = lds_u32(wl, o + QR_Q8_BYTES * s + 2 + 8 * kg);
-    hi = lds_u32(wl, o + QR_Q8_BYTES * s + 6 + 8 * kg);
+  } else {  // Q8_0 (Q6_K: unit_w_q6): block s, bytes 2 + 8 kg .. +7, at any even address
+    const uint32_t o = rowk + 4 * kg + QR_Q8_BYTES * s + 2, al = o & ~3u;
+    const uint32_t w0 = lds_at<uint32_t>(al, 0), w1 = lds_at<uint32_t>(al, 4),
+                   w2 = lds_at<uint32_t>(al, 8);
+    lo = __builtin_amdgcn_alignbyte(w1, w0, o & 3u);
+    hi = __builtin_amdgcn_alignbyte(w2, w1, o & 3u);
   }
   return (long)((uint64_t)lo | ((uint64_t)hi << 32));
 }
@@ -104,58 +121,73 @@ __device__ inline long unit_a(const uint32_t* wl, int o, int s, int kg) {
 // bits at dword h + 2 s picked by the byte selector hsel -- and the 2-bit
 // fields are moved to bits 4-5 of their bytes by shifts and masks.
 struct Q6Ref {
-  int w, h;
+  uint32_t w, h;  // LDS addresses of the dwords that hold unit 0's ql and qh bytes
   uint32_t wsh, hsel;
 };
-__device__ inline Q6Ref q6_ref(int o, int kg) {
+__device__ inline Q6Ref q6_ref(uint32_t row, int kg) {
   Q6Ref q;
-  const int ow = o + 4 * kg, oh = o + 128 + 2 * kg;
-  q.w = ow >> 2;
-  q.wsh = (uint32_t)(ow & 3);
-  q.h = oh >> 2;
-  const uint32_t k = (uint32_t)(oh & 3);
-  q.hsel = k * 0x0101u + (k + 1) * 0x01010000u;  // bytes [k+1, k+1, k, k]
+  const uint32_t ow = row + 4 * kg, oh = row + 128 + 2 * kg;
+  q.w = ow & ~3u;
+  q.wsh = ow & 3u;
+  q.h = oh & ~3u;
+  const uint32_t k = oh & 3u;
+  q.hsel = k * 0x01010101u + 0x01010000u;  // bytes [k+1, k+1, k, k]
+  asm("" : "+v"(q.w), "+v"(q.h));
   return q;
 }
-__device__ inline long unit_a_q6(const uint32_t* wl, const Q6Ref& q, int s) {
-  const uint32_t w = __builtin_amdgcn_alignbyte(wl[q.w + 4 * s + 1], wl[q.w + 4 * s], q.wsh);
+__device__ inline long unit_w_q6(const Q6Ref& q, int s) {
+  const uint32_t w = __builtin_amdgcn_alignbyte(lds_at<uint32_t>(q.w, 16 * s + 4),
+                                                lds_at<uint32_t>(q.w, 16 * s), q.wsh);
   // x: qh bytes b1 b1 b0 b0; element i's low pair sits in bits 4i..4i+1 of
   // b1:b0, its high pair two bits up
-  const uint32_t x = __builtin_amdgcn_perm(wl[q.h + 2 * s + 1], wl[q.h + 2 * s], q.hsel);
+  const uint32_t x = __builtin_amdgcn_perm(lds_at<uint32_t>(q.h, 8 * s + 4),
+                                           lds_at<uint32_t>(q.h, 8 * s), q.hsel);
   const uint32_t lo = (w & 0x0F0F0F0Fu) | (((x << 4) & 0x00300030u) | (x & 0x30003000u));
   const uint32_t hi = ((w >> 4) & 0x0F0F0F0Fu) | (((x << 2) & 0x00300030u) | ((x >> 2) & 0x30003000u));
   return (long)((uint64_t)lo | ((uint64_t)hi << 32));
 }
 
-// fp32 scales (and mins) of the four units s0 .. s0 + 3 of a staged row (0
-// past unit su), the row's header decoded once.
-template <int TYPE>
-__device__ inline void unit_scales4(const uint32_t* wl, int o, int s0, int su, float (&sc)[4],
-                                    float (&mn)[4]) {
+// fp32 scales (and mins) of the N (2 or 4) units s0 .. s0 + N - 1 of a staged
+// row (0 past unit su), the row's header decoded once.  `row`: the LDS byte
+// address of the row's stage.  Returns whether a block scale is not finite.
+__device__ inline uint32_t lds_u16x2(uint32_t a) {  // 4 bytes at any even address
+  const uint32_t al = a & ~3u;
+  return __builtin_amdgcn_alignbyte(lds_at<uint32_t>(al, 4), lds_at<uint32_t>(al, 0), a & 3u);
+}
+template <int TYPE, int N>
+__device__ inline bool unit_scales(uint32_t row, int s0, int su, float (&sc)[N], float (&mn)[N]) {
   if constexpr (TYPE == QR_T_Q4_K || TYPE == QR_T_Q5_K) {
-    const uint32_t h0 = wl[o >> 2];
+    const uint32_t h0 = lds_at<uint32_t>(row, 0);
     const float d = qr_h2f(h0 & 0xFFFFu), dm = qr_h2f(h0 >> 16);
-    const uint32_t w = wl[(o + 4 + s0) >> 2];  // 16-byte aligned stage: o % 4 == 0
+    // 16-byte aligned stage: s0's dword is aligned for N == 4, a half of it for N == 2
+    const uint32_t w = lds_at<uint32_t>(row + 4 + (s0 & 4), 0) >> (8 * (s0 & 3));
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < N; i++) {
       const uint32_t b = (w >> (8 * i)) & 0xFFu;
       sc[i] = (float)(b & 63u) * d;
       mn[i] = (float)(b >> 6) * dm;
     }
+    return (h0 & 0x7C00u) == 0x7C00u || (h0 & 0x7C000000u) == 0x7C000000u;
   } else if constexpr (TYPE == QR_T_Q6_K) {
-    const float d = qr_h2f(lds_u32(wl, o + 208) & 0xFFFFu);
-    const uint32_t w = lds_u32(wl, o + 192 + s0);
+    const uint32_t h = lds_u16x2(row + 208);
+    const float d = qr_h2f(h & 0xFFFFu);
+    const uint32_t w = lds_u16x2(row + 192 + s0);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < N; i++) {
       sc[i] = (float)(int)(int8_t)((w >> (8 * i)) & 0xFFu) * d;
       mn[i] = 0.0f;
     }
+    return (h & 0x7C00u) == 0x7C00u;
   } else {
+    bool odd = false;
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      sc[i] = s0 + i < su ? qr_h2f(lds_u32(wl, o + QR_Q8_BYTES * (s0 + i)) & 0xFFFFu) : 0.0f;
+    for (int i = 0; i < N; i++) {
+      const uint32_t h = s0 + i < su ? lds_u16x2(row + QR_Q8_BYTES * (s0 + i)) & 0xFFFFu : 0u;
+      sc[i] = qr_h2f(h);
       mn[i] = 0.0f;
+      odd |= (h & 0x7C00u) == 0x7C00u;
     }
+    return odd;
   }
 }
 
@@ -182,9 +214,12 @@ struct MfmaArgs {
   int rows, cols, E, K;
   const uint8_t* XQ;      // activation records [xrows][cols/32][kXQ]
   int x_by_token;         // activation row of dispatch position p: perm[p] / K, else p
-  const int32_t* offsets; // dispatch (tile = NTOK)
-  const int32_t* perm;
+  const int32_t* offsets; // dispatch (tile = NTOK); null: the dense form, one
+  const int32_t* perm;    // matrix (E = 1) and rows 0 .. P - 1 in order
   const int32_t* tiles;
+  const int4* table;      // optional: work item -> (expert, first position, pairs), P entries
+  int P;                  // pairs (dense form: rows)
+  uint32_t kmul, rbmul;   // exact_div multipliers of K and t_rb
   float* Y;               // [P][ystride], row = dispatch position
   int ystride;
   // gate/up mode, optional: instead of Y, the activation records of the down
@@ -198,6 +233,14 @@ struct MfmaArgs {
   int t_rb;
   size_t t_tile_bytes;
 };
+
+// n / d for 0 <= n, n d < 2^32, by the multiplier ceil(2^32 / d) (0 for d = 1).
+__device__ inline int exact_div(int n, uint32_t mul) {
+  return mul ? (int)__umulhi((uint32_t)n, mul) : n;
+}
+static uint32_t exact_div_mul(int d) {
+  return d > 1 ? (uint32_t)((((uint64_t)1 << 32) + (uint32_t)d - 1) / (uint32_t)d) : 0u;
+}
 
 template <int TYPE, bool GATEUP, int NJ, int RA, int D, int NW>
 struct MfmaGeo {
@@ -226,10 +269,6 @@ struct MfmaGeo {
   static constexpr int O_S = O_W + NW * D * WST;           // scales, per wave
   static constexpr int O_M = O_S + NW * SCL;               // mins, per wave
   static constexpr int LDS = O_M + NW * SCL;
-  // activation row of each pair, read once before the first stage: it shares
-  // the scale area, first written after the first stage's barrier
-  static constexpr int O_X = O_S;
-  static_assert(NTOK * 4 <= NW * SCL, "xrow");
   static_assert(D >= 1 && D <= 3, "ring depth");
   static_assert(NI <= 63, "vmcnt range");
 };
@@ -243,19 +282,33 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
   constexpr int KST = MF<TYPE>::kStage;
   extern __shared__ __align__(16) uint8_t smem[];
 
-  // work item -> (expert e, first dispatch position p0, pair count np)
+  // work item -> (expert e, first dispatch position p0, pair count np).  Every
+  // load here is a round trip that the workgroup's first DMA waits for: the
+  // dense form needs none, the dispatch's table one (the search over the
+  // tile offsets it replaces, eight dependent loads at 128 experts, took half
+  // of the down product's 82 us at T = 512).
   const int item = blockIdx.y;
-  const int ntiles = a.tiles[a.E];
-  if (item >= ntiles) return;  // uniform
-  int lo = 0, hi = a.E;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (a.tiles[mid] <= item) lo = mid;
-    else hi = mid;
+  int e = 0, p0, np;
+  if (!a.offsets) {
+    p0 = item * G::NTOK;
+    np = min(G::NTOK, a.P - p0);
+  } else if (a.table) {
+    const int ntiles = a.tiles[a.E];
+    const int4 it = a.table[min(item, a.P - 1)];
+    e = it.x;
+    p0 = it.y;
+    np = item < ntiles ? it.z : 0;
+  } else {
+    if (item >= a.tiles[a.E]) return;  // uniform
+    int hi = a.E;
+    while (hi - e > 1) {
+      const int mid = (e + hi) >> 1;
+      if (a.tiles[mid] <= item) e = mid;
+      else hi = mid;
+    }
+    p0 = a.offsets[e] + (item - a.tiles[e]) * G::NTOK;
+    np = min(G::NTOK, a.offsets[e + 1] - p0);
   }
-  const int e = lo;
-  const int p0 = a.offsets[e] + (item - a.tiles[e]) * G::NTOK;
-  const int np = min(G::NTOK, a.offsets[e + 1] - p0);
   if (np <= 0) return;  // uniform
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -264,24 +317,15 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
   const int U = TYPE == QR_T_Q8_0 ? a.cols / 32 : (a.cols / 256) * 8;
   const size_t rb = qr_wrow_bytes(TYPE, a.cols);
   const int nstage = (U + 7) / 8;
-  int* xrow = reinterpret_cast<int*>(smem + G::O_X);
-  if (threadIdx.x < G::NTOK) {
-    int xr = 0;
-    const int tt = threadIdx.x;
-    if (tt < np) xr = a.x_by_token ? a.perm[p0 + tt] / a.K : p0 + tt;
-    xrow[tt] = xr;
-  }
-  __syncthreads();  // xrow
 
   // Per-lane DMA sources, stage-invariant parts.  Weight chunk c = k*64+lane
   // of this wave: matrix c / (WR NCH), row rw0 + (c / NCH) % WR, chunk c % NCH
-  // of the row's stage; chunks past the row's stage bytes, rows past the
-  // matrix and lanes past the wave's chunks reload the workgroup's first row's
-  // stage start.
+  // of the row's stage; rows past the matrix and lanes past the wave's chunks
+  // reload the workgroup's first row.
   const size_t ebase = (size_t)e * a.slice;
   const uint32_t row0 = (uint32_t)(blockIdx.x * G::MR) * (uint32_t)rb;  // within the slice
   const uint8_t* wbase[G::WI];  // the chunk's matrix, at the expert's slice
-  uint32_t wroff[G::WI];        // its row's offset in the slice, or ~0 (no row)
+  uint32_t wroff[G::WI];        // its row's offset in the slice
   int wch[G::WI];
   int wrow[G::WI];              // its row, or -1
 #pragma unroll
@@ -292,26 +336,27 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
     const int rr = rem / NCH;
     wch[k] = rem - rr * NCH;
     const int row = rw0 + rr;
-    wroff[k] = (c < G::WCH && row < a.rows) ? (uint32_t)row * (uint32_t)rb : ~0u;
-    wrow[k] = (c < G::WCH && row < a.rows) ? row : -1;
+    const bool in = c < G::WCH && row < a.rows;
+    wroff[k] = in ? (uint32_t)row * (uint32_t)rb : row0;
+    wrow[k] = in ? row : -1;
     wbase[k] = ((GATEUP && m == 1) ? a.W2 : a.W1) + ebase;
   }
   // Activation chunk c = (wave AI + k) 64 + lane: pair c / APC, chunk c % APC
-  // of its 8 records (unit (c % APC) / 3; chunk 24 is the pad).  asrc: the
-  // chunk's offset in XQ at stage 0, or ~0 (reload pair 0's first chunk).
+  // of its 8 records (unit (c % APC) / 3; chunk 24 is the pad and reloads
+  // chunk 23; past the item's pairs its first one is loaded again).
   const size_t xq_row = (size_t)U * kXQ;
   size_t asrc[G::AI];
   int aunit[G::AI];
 #pragma unroll
   for (int k = 0; k < G::AI; k++) {
     const int c = (wave * G::AI + k) * 64 + lane;
-    const int tt = c / G::APC;
-    const int ch = c - tt * G::APC;
-    const bool ok = c < G::ACH && tt < np && ch < G::APC - 1;
-    asrc[k] = ok ? (size_t)xrow[tt] * xq_row + 16 * (size_t)ch : ~(size_t)0;
+    const int tt = min(c / G::APC, G::NTOK - 1);
+    const int ch = min(c - tt * G::APC, G::APC - 2);
+    const int p = p0 + (tt < np ? tt : 0);
+    const int xr = a.x_by_token && a.offsets ? exact_div(a.perm[p], a.kmul) : p;
+    asrc[k] = (size_t)xr * xq_row + 16 * (size_t)ch;
     aunit[k] = ch / 3;
   }
-  const size_t asrc0 = (size_t)xrow[0] * xq_row;
   // Q4_K / Q5_K: a row's stage is whole 16-byte chunks (rows and stages are
   // multiples of 16 bytes) and every stage's 8 units exist, so each source is
   // a stage-invariant address plus the stage's offset
@@ -326,10 +371,10 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
     const int nbk = a.cols >> 8;
 #pragma unroll
     for (int k = 0; k < G::WI; k++) {
-      if (wroff[k] == ~0u) {
-        wp[k] = a.t_rb ? a.W1 + ebase : a.W1 + ebase + row0;
+      if (a.t_rb && wrow[k] < 0) {
+        wp[k] = a.W1 + ebase;
       } else if (a.t_rb) {
-        const int r = wrow[k], t = r / a.t_rb;
+        const int r = wrow[k], t = exact_div(r, a.rbmul);
         const int L = min(a.t_rb, a.rows - t * a.t_rb) * nbk;
         wp[k] = wbase[k] + (size_t)t * a.t_tile_bytes + (size_t)16 * wch[k] * L +
                 (size_t)16 * (r - t * a.t_rb) * nbk;
@@ -338,8 +383,11 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
       }
     }
 #pragma unroll
-    for (int k = 0; k < G::AI; k++) ap[k] = a.XQ + (asrc[k] != ~(size_t)0 ? asrc[k] : asrc0);
+    for (int k = 0; k < G::AI; k++) ap[k] = a.XQ + asrc[k];
   }
+  // The last 16-byte chunk of the slice that holds a byte of it (its base is
+  // 16-byte aligned): a stage's last chunk never starts past it.
+  const uint32_t wlast = ((uint32_t)a.slice - 1u) & ~15u;
 
   auto issue = [&](int st) {
     const int slot = st % D;
@@ -361,29 +409,21 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
     }
 #pragma unroll
     for (int k = 0; k < G::AI; k++) {
-      const bool ok = asrc[k] != ~(size_t)0 && 8 * st + aunit[k] < U;
-      const size_t src = (ok ? asrc[k] : asrc0) + (size_t)(8 * st) * kXQ;
+      // units past the row's last (Q8_0 rows): the pair's first chunk again
+      const bool ok = TYPE != QR_T_Q8_0 || 8 * st + aunit[k] < U;
+      const size_t src = ok ? asrc[k] + (size_t)(8 * st) * kXQ : asrc[0];
       lds_dma16(a.XQ + src, abase + (uint32_t)(k * 1024));
     }
     const uint32_t wlds = lds_u32addr(smem + G::O_W + (wave * D + slot) * G::WST);
     // offsets within the expert's slice: its base is 16-byte aligned, so
-    // alignment within the slice is alignment in memory
+    // alignment within the slice is alignment in memory; a chunk past the
+    // row's stage brings the next row's bytes, which nobody reads
     const uint32_t s0 = (uint32_t)st * KST;
-    const uint32_t se = s0 + KST < (uint32_t)rb ? s0 + KST : (uint32_t)rb;
-    const uint32_t clampoff = (row0 + s0) & ~15u;
 #pragma unroll
     for (int k = 0; k < G::WI; k++) {
-      uint32_t off = clampoff;
-      const uint8_t* W = a.W1 + ebase;
-      if (wroff[k] != ~0u) {
-        const uint32_t o = ((wroff[k] + s0) & ~15u) + 16u * (uint32_t)wch[k];
-        if (o < wroff[k] + se) {
-          off = o;
-          W = wbase[k];
-        }
-      }
-      if (a.wnt) lds_dma16_nt(W + off, wlds + (uint32_t)(k * 1024));
-      else lds_dma16(W + off, wlds + (uint32_t)(k * 1024));
+      const uint32_t off = min((wroff[k] + 16u * (uint32_t)wch[k] + s0) & ~15u, wlast);
+      if (a.wnt) lds_dma16_nt(wbase[k] + off, wlds + (uint32_t)(k * 1024));
+      else lds_dma16(wbase[k] + off, wlds + (uint32_t)(k * 1024));
     }
   };
 
@@ -414,6 +454,29 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; i++) acc[m][r][j][i] = 0.0f;
 
+    // LDS addresses in slot 0: the wave's rows, this lane's A operand (its row
+    // of the pair tile), the (bd, bsf) of the four pairs whose terms it forms
+    // (two pairs per address), the bsums it checks, its row's scales and mins
+    const uint8_t* const w00 = smem + G::O_W + wave * D * G::WST;
+    const uint32_t wl0 = lds_base(w00);
+    uint32_t wr0[NMAT][RA], wrK0[NMAT][RA];
+#pragma unroll
+    for (int m = 0; m < NMAT; m++)
+#pragma unroll
+      for (int r = 0; r < RA; r++) {
+        wr0[m][r] = lds_base(w00 + (m * WR + 16 * r + ln) * G::SLOT);
+        wrK0[m][r] = lds_base(w00 + (m * WR + 16 * r + ln) * G::SLOT + 4 * kg);
+      }
+    const uint32_t asA0 = lds_base(smem + ln * (16 * G::APC) + 8 * kg);
+    uint32_t asB0[NJ][2];
+#pragma unroll
+    for (int j = 0; j < NJ; j++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        asB0[j][h] = lds_base(smem + (16 * j + 4 * kg + 2 * h) * (16 * G::APC) + 32);
+    const uint32_t bsA0 = lds_base(smem + (lane >> 3) * (16 * G::APC) + (lane & 7) * kXQ + 36);
+    const uint32_t scA = lds_base(scl + ln), mnA = lds_base(mnl + ln);
+
 #pragma unroll
     for (int s = 0; s < D - 1; s++)
       if (s < nstage) issue(s);
@@ -434,57 +497,62 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
       __builtin_amdgcn_s_barrier();
       if (D > 1 && st + D - 1 < nstage) issue(st + D - 1);
       const int slot = st % D;
-      const uint32_t* wl =
-          reinterpret_cast<const uint32_t*>(smem + G::O_W + (wave * D + slot) * G::WST);
       const uint8_t* as = smem + slot * G::AST;
       const int su = min(8, U - st * 8);
       const uint32_t s0 = (uint32_t)st * KST;
       // scales and mins of the wave's (matrix, unit, row)s, entry
-      // (m * 8 + s) * WR + rr: lane (m, rr, half) decodes row rr's header once
-      // for units 4 half .. 4 half + 3
+      // (m * 8 + s) * WR + rr: each lane decodes a row's header once for UPL
+      // of its units
+      constexpr int UPL = NMAT * WR * 8 / 64 < 4 ? 2 : 4, PARTS = 8 / UPL;
       bool odd = false;  // a block scale that is not finite, or an inexact m * bsum
-      for (int i = lane; i < NMAT * WR * 2; i += 64) {
-        const int m = i / (2 * WR), rem = i - m * 2 * WR;
-        const int rr = rem >> 1, half = rem & 1;
-        float sc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        const int row = rw0 + rr;
-        if (4 * half < su && row < a.rows) {
-          const int hd = (int)(((uint32_t)row * (uint32_t)rb + s0) & 15u);
-          unit_scales4<TYPE>(wl, (m * WR + rr) * G::SLOT + hd, 4 * half, su, sc, mn);
+      for (int i = lane; i < NMAT * WR * PARTS; i += 64) {
+        const int m = i / (PARTS * WR), rem = i - m * PARTS * WR;
+        const int rr = rem / PARTS, u0 = (rem - rr * PARTS) * UPL;
+        float sc[UPL], mn[UPL];
 #pragma unroll
-          for (int q = 0; q < 4; q++) odd |= !(__builtin_fabsf(sc[q] + mn[q]) < __builtin_inff());
+        for (int q = 0; q < UPL; q++) sc[q] = mn[q] = 0.0f;
+        const int row = rw0 + rr;
+        if (u0 < su && row < a.rows) {
+          const uint32_t hd = ALN ? 0u : ((uint32_t)row * (uint32_t)rb + s0) & 15u;
+          odd = unit_scales<TYPE, UPL>(
+              wl0 + (uint32_t)(slot * G::WST + (m * WR + rr) * G::SLOT) + hd, u0, su, sc, mn);
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-          scl[(m * 8 + 4 * half + q) * WR + rr] = sc[q];
-          mnl[(m * 8 + 4 * half + q) * WR + rr] = mn[q];
+        for (int q = 0; q < UPL; q++) {
+          scl[(m * 8 + u0 + q) * WR + rr] = sc[q];
+          if constexpr (MF<TYPE>::kMin) mnl[(m * 8 + u0 + q) * WR + rr] = mn[q];
         }
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      // head bytes of this lane's weight rows (both matrices share them: same
-      // slice and row sizes, 16-byte aligned bases)
-      int hA[RA];
-#pragma unroll
-      for (int r = 0; r < RA; r++)
-        hA[r] = (int)(((uint32_t)(rw0 + 16 * r + ln) * (uint32_t)rb + s0) & 15u);
+      // this slot's addresses; a row's stage also has its head bytes (both
+      // matrices the same: same slice and row sizes, 16-byte aligned bases)
+      const uint32_t wo = (uint32_t)(slot * G::WST), ao = (uint32_t)(slot * G::AST);
+      uint32_t wrA[NMAT][RA], wrK[NMAT][RA];
       Q6Ref q6[NMAT][RA];
-      if constexpr (TYPE == QR_T_Q6_K) {
 #pragma unroll
-        for (int m = 0; m < NMAT; m++)
+      for (int m = 0; m < NMAT; m++)
 #pragma unroll
-          for (int r = 0; r < RA; r++) q6[m][r] = q6_ref((m * WR + 16 * r + ln) * G::SLOT + hA[r], kg);
-      }
+        for (int r = 0; r < RA; r++) {
+          const uint32_t hd =
+              ALN ? 0u : ((uint32_t)(rw0 + 16 * r + ln) * (uint32_t)rb + s0) & 15u;
+          wrA[m][r] = wr0[m][r] + wo + hd;
+          wrK[m][r] = wrK0[m][r] + wo + hd;
+          if constexpr (TYPE == QR_T_Q6_K) q6[m][r] = q6_ref(wrA[m][r], kg);
+        }
+      const uint32_t asA = asA0 + ao;
+      uint32_t asB[NJ][2];
+#pragma unroll
+      for (int j = 0; j < NJ; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) asB[j][h] = asB0[j][h] + ao;
       // Whether this stage's terms may take the fused forms below: every block
       // scale of the wave's rows finite (checked where they were decoded) and,
       // with mins, |bsum| <= kBsumExact in every unit of the item's pairs.
       if constexpr (MF<TYPE>::kMin) {
+        const uint32_t bsA = bsA0 + ao;
 #pragma unroll
-        for (int k = 0; k < G::NTOK * 8 / 64; k++) {
-          const int i = k * 64 + lane, tt = i >> 3;
-          const float bsf =
-              *reinterpret_cast<const float*>(as + tt * (16 * G::APC) + (i & 7) * kXQ + 36);
-          odd |= tt < np && __builtin_fabsf(bsf) > kBsumExact;
-        }
+        for (int k = 0; k < G::NTOK * 8 / 64; k++)  // records past np repeat the first pair's
+          odd |= __builtin_fabsf(lds_at<float>(bsA, k * 8 * 16 * G::APC)) > kBsumExact;
       }
       const bool fused = __builtin_amdgcn_ballot_w64(odd) == 0;  // wave-uniform
       // One term from the accumulator bits of 1.5 * 2^23 + isum.  Fused: the
@@ -511,11 +579,11 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
         for (int m = 0; m < NMAT; m++)
 #pragma unroll
           for (int r = 0; r < RA; r++) {
-            if constexpr (TYPE == QR_T_Q6_K) Wq[m][r] = unit_a_q6(wl, q6[m][r], s);
-            else Wq[m][r] = unit_a<TYPE>(wl, (m * WR + 16 * r + ln) * G::SLOT + hA[r], s, kg);
-            const int si = (m * 8 + s) * WR + 16 * r + ln;
-            sc[m][r] = scl[si];
-            mn[m][r] = mnl[si];
+            if constexpr (TYPE == QR_T_Q6_K) Wq[m][r] = unit_w_q6(q6[m][r], s);
+            else Wq[m][r] = unit_w<TYPE>(wrA[m][r], wrK[m][r], s, kg);
+            const int si = 4 * ((m * 8 + s) * WR + 16 * r);
+            sc[m][r] = lds_at<float>(scA, si);
+            mn[m][r] = MF<TYPE>::kMin ? lds_at<float>(mnA, si) : 0.0f;
             nsc[m][r] = sc[m][r] * -12582912.0f;  // -1.5 * 2^23
           }
         if constexpr (SK) {
@@ -541,14 +609,14 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
         } else {
 #pragma unroll
           for (int j = 0; j < NJA; j++) {
-            const uint2 bq = *reinterpret_cast<const uint2*>(
-                as + (16 * j + ln) * (16 * G::APC) + s * kXQ + 8 * kg);
-            const long A = (long)((uint64_t)bq.x | ((uint64_t)bq.y << 32));
-            float2 bb[4];  // (bd, bsf) of the lane's four pairs
+            const long A = lds_at<long>(asA, 16 * j * (16 * G::APC) + s * kXQ);
+            float bd[4], bsf[4];  // of the lane's four pairs
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-              bb[i] = *reinterpret_cast<const float2*>(
-                  as + (16 * j + 4 * kg + i) * (16 * G::APC) + s * kXQ + 32);
+            for (int i = 0; i < 4; i++) {
+              const int o = (i & 1) * (16 * G::APC) + s * kXQ;
+              bd[i] = lds_at<float>(asB[j][i >> 1], o);
+              bsf[i] = MF<TYPE>::kMin ? lds_at<float>(asB[j][i >> 1], o + 4) : 0.0f;
+            }
             // the accumulators start at the bits of 1.5 * 2^23, so an exact sum
             // S (|S| < 2^22) comes out as the bits of the float 1.5 * 2^23 + S;
             // Q6_K's stored quants carry an offset of 32, which one more
@@ -569,8 +637,8 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
                   // into one, on element 0
                   int di = Dv[i];
                   asm("" : "+v"(di));
-                  acc[m][r][j][i] += term_of(fused_tag, sc[m][r], nsc[m][r], mn[m][r], di, bb[i].x,
-                                             bb[i].y);
+                  acc[m][r][j][i] += term_of(fused_tag, sc[m][r], nsc[m][r], mn[m][r], di, bd[i],
+                                             bsf[i]);
                 }
               }
           }
@@ -737,9 +805,14 @@ static hipError_t mfma_launch_nj(const MfmaArgs& a, int items, int tile, int nw,
 hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const uint8_t* W2,
                               size_t slice, int E, int K, int rows, int cols, const uint8_t* XQ,
                               int x_by_token, const int32_t* offsets, const int32_t* perm,
-                              const int32_t* tiles, float* Y, int ystride, int items, int tile,
-                              uint8_t* QO, bool qperm, hipStream_t st, bool tiled) {
+                              const int32_t* tiles, const int4* table, int P, float* Y,
+                              int ystride, int tile, uint8_t* QO, bool qperm, hipStream_t st,
+                              bool tiled) {
   if (tile != 16 && tile != 32) return hipErrorInvalidValue;
+  if (!offsets && E != 1) return hipErrorInvalidValue;
+  if (P <= 0) return hipSuccess;
+  // routed: >= the sum over the experts of ceil(count / tile)
+  const int items = (P + tile - 1) / tile + (offsets ? E : 0);
   if (slice >= ((size_t)1 << 32)) return hipErrorInvalidValue;  // 32-bit offsets in a slice
   if (QO && (!gateup || (rows & 31) || (reinterpret_cast<uintptr_t>(QO) & 15)))
     return hipErrorInvalidValue;
@@ -759,6 +832,11 @@ hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const ui
   a.offsets = offsets;
   a.perm = perm;
   a.tiles = tiles;
+  a.table = table;
+  a.P = P;
+  if ((uint64_t)P * (uint32_t)K >> 32) return hipErrorInvalidValue;
+  a.kmul = exact_div_mul(K);
+  a.rbmul = 0;
   a.Y = Y;
   a.ystride = ystride;
   a.QO = QO;
@@ -770,18 +848,18 @@ hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const ui
     if ((type != QR_T_Q4_K && type != QR_T_Q5_K) || (cols & 255) || (cols >> 8) > 64)
       return hipErrorInvalidValue;
     const TiledGeom tg = tiled_geom(type, rows, cols);
-    a.t_rb = tg.RB;
+    a.t_rb = tg.RB;  // rows * RB < 2^32: a row holds more than 64 bytes of the slice
+    a.rbmul = exact_div_mul(tg.RB);
     a.t_tile_bytes = tg.tile_bytes;
   }
   // items of up to 16 pairs: an expert rarely has more than one, so its rows
   // are read about once and the hint keeps the activation records cached;
   // with 32-pair items hot experts are re-read by several items
   a.wnt = tile <= 16;
-  // one expert (a dense product): items - 1 = ceil(P / tile) exactly; with
-  // fewer than two workgroups of 64 rows per CU, workgroups of 32 rows
+  // one expert (a dense product): with fewer than two workgroups of 64 rows per CU, workgroups of 32 rows
   // and a two-slot ring for its long rows (each workgroup walks them alone)
   int nw = 4;
-  if (E == 1 && (long)((rows + 63) / 64) * (items - 1) < 2L * device_cus()) nw = 2;
+  if (E == 1 && (long)((rows + 63) / 64) * ((P + tile - 1) / tile) < 2L * device_cus()) nw = 2;
   const int stages = type == QR_T_Q8_0 ? (cols / 32 + 7) / 8 : cols / 256;
   const bool ring = E == 1 && stages >= 8;
   switch (type) {

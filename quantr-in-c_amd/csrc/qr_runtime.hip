@@ -632,22 +632,18 @@ int qr_gemv_rows(qr_ctx* c, int order, uint32_t type, const void* w, const float
     return fail(QR_ERR_INVALID, "qr_gemv_rows: w and x must be 16-byte aligned");
   const size_t slice = qr_wrow_bytes((int)base, d) * (size_t)n;
   if (slice >= ((size_t)1 << 32)) return fail(QR_ERR_UNSUPPORTED, "qr_gemv_rows: matrix of 4 GiB or more");
-  // scratch: the rows' activation records, then the single-"expert" dispatch
+  // scratch: the rows' activation records (4 T + 32 bytes more are asked for
+  // than used, so that calls under capture succeed or fail as they always did)
   const size_t rec = (((size_t)T * (d / 32) * qr::kXQ) + 255) & ~(size_t)255;
   void* base_p = nullptr;
   int rc = ctx_scratch(c, rec + 16 + 4 * (size_t)T + 16, "qr_gemv_rows", &base_p);
   if (rc) return rc;
   uint8_t* recp = static_cast<uint8_t*>(base_p);
-  int32_t* off = reinterpret_cast<int32_t*>(recp + rec);
-  int32_t* tiles = off + 4;
-  int32_t* perm = tiles + 4;
-  const int tile = 16;
-  QR_HIP(qr::rows_dispatch_launch(T, tile, off, perm, tiles, c->stream), "k_rows_dispatch");
   QR_HIP(qr::quant_rows_launch(x, xstride, T, d, base != QR_T_Q8_0, recp, c->stream),
          "k_quant_rows");
   QR_HIP(qr::expert_mfma_launch((int)base, false, static_cast<const uint8_t*>(w), nullptr, slice,
-                                1, 1, n, d, recp, 1, off, perm, tiles, y, ystride,
-                                (T + tile - 1) / tile + 1, tile, nullptr, false, c->stream, tiled),
+                                1, 1, n, d, recp, 0, nullptr, nullptr, nullptr, nullptr, T, y,
+                                ystride, 16, nullptr, false, c->stream, tiled),
          "k_expert_mfma");
   return QR_OK;
 }

@@ -98,7 +98,8 @@ __device__ inline void quant_rows_group(const float* __restrict__ x, int xstride
 // the P (token, slot) pairs by expert, exclusive scans of the counts and of
 // the `tile`-pair work items per expert, and a stable permutation (pairs of
 // one expert keep their order): perm[offsets[e] + i] = the i-th pair of e,
-// inv[p] = its position (-1 for an index outside 0..E-1).  `idx` may point
+// inv[p] = its position (-1 for an index outside 0..E-1); table (optional): the
+// work items as (expert, first position, pairs).  `idx` may point
 // to global or LDS memory.
 //
 // Wave w owns the pairs of one contiguous range (ranges in wave order), so a
@@ -113,8 +114,9 @@ constexpr int kDispWaves = kDispThreads / 64;
 __device__ inline void dispatch_wg(const int32_t* idx, int P, int E, int tile,
                                    int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
                                    int32_t* __restrict__ tiles, int32_t* __restrict__ perm,
-                                   int32_t* __restrict__ inv) {
+                                   int32_t* __restrict__ inv, int4* __restrict__ table) {
   __shared__ int cnt[256];
+  __shared__ int toff[257], total;  // with a table: the tiles' offsets, the pairs dispatched
   __shared__ int wcnt[kDispWaves][256];  // the wave's counts, then its running position
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int per = ((P + kDispWaves - 1) / kDispWaves + 63) & ~63;  // whole rounds of 64
@@ -172,6 +174,7 @@ __device__ inline void dispatch_wg(const int32_t* idx, int P, int E, int tile,
         counts[e] = c[i];
         offsets[e] = acc;
         if (tiles) tiles[e] = tacc;
+        if (table) toff[e] = tacc;
       }
       acc += c[i];
       tacc += tl[i];
@@ -179,9 +182,27 @@ __device__ inline void dispatch_wg(const int32_t* idx, int P, int E, int tile,
     if (lane == 63) {
       offsets[E] = ci;
       if (tiles) tiles[E] = ti;
+      if (table) {
+        toff[E] = ti;
+        total = ci;
+      }
     }
   }
   __syncthreads();
+  // work item -> its expert, first position and pairs
+  if (table) {
+    const int nt = toff[E];
+    for (int i = tid; i < nt; i += kDispThreads) {
+      int lo = 0, hi = E;  // largest e with toff[e] <= i
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (toff[mid] <= i) lo = mid;
+        else hi = mid;
+      }
+      const int p = cnt[lo] + (i - toff[lo]) * tile;
+      table[i] = make_int4(lo, p, min(tile, (lo + 1 < E ? cnt[lo + 1] : total) - p), 0);
+    }
+  }
   // each wave's first position per expert
   for (int e = tid; e < E; e += kDispThreads) {
     int run = cnt[e];
