@@ -896,6 +896,8 @@ bool gemv_ggml_ok(int type, int d, int nt) {
   return ggml_lds_bytes(type, d, n4, ggml_xm(type, d, n4)) <= kLdsMax;
 }
 
+// pairs: rows of workgroups (grid y), one per pair (GemvArgs::eidx) or per NT
+// tokens; 0: one
 template <int T, int NT, int XM, int G = 1>
 static hipError_t launch_ggml_x(const GemvArgs& a, hipStream_t st, int pairs = 0) {
   static std::atomic<bool> opted[64];
@@ -914,7 +916,7 @@ static hipError_t launch_ggml_x(const GemvArgs& a, hipStream_t st, int pairs = 0
   // workgroups per CU, not the four its LDS allows)
   per_cu = std::min(per_cu, resident_by_regs((const void*)k_gemv_ggml<T, NT, XM, G>, 256, by_regs));
   const int want = (ntiles + 3) / 4;
-  // pair mode: the pairs' matrices share the resident workgroups
+  // the rows share the resident workgroups
   const int cap = pairs > 0 ? (device_cus() * per_cu + pairs - 1) / pairs : device_cus() * per_cu;
   // as few rounds of the resident grid as the tiles need, the tiles spread
   // evenly over them (every wave the same number of tiles, give or take one)
@@ -938,20 +940,31 @@ static hipError_t launch_ggml_t(const GemvArgs& a, hipStream_t st, int pairs = 0
                           : launch_ggml_x<T, NT, kXmLate>(a, st, pairs);
 }
 
+// Several tokens: each token its own row of workgroups (grid y), or several
+// per workgroup, sharing the decoding of the weights.  A lane computes a whole
+// super-block, so one token's pass leaves a wave a long serial piece that more
+// tokens per wave only lengthen, while the matrix's second reader finds it in
+// the caches.  Single tokens wherever one token's tiles are at most three
+// workgroups per CU (Q4_K / Q5_K / Q6_K: 5632 x 2048, three tokens, 14.6 / 14.3 /
+// 17.1 us together, 6.8 / 7.6 / 15.6 apart; 2048 x 5632, eight, 74 / 75 / 82
+// against 24 / 26 / 34; 12000 x 3072, four, 33 / 35 / 44 against 19 / 24 / 35).
+// Beyond that only Q4_K's cheap decoding stands the repetition (32000 x 2048,
+// four tokens: 27.2 together, 25.6 apart; Q5_K 28.8 and 32.2, Q6_K 38.3 and
+// 49.3), and eight tokens are two rows of four in one launch (32000 x 2048:
+// 41.4 / 44.2 / 63.9 us; apart 48.9 / 59.2 / 88.1; one after the other
+// 54.3 / 57.7 / 76.6).
 template <int T>
 static hipError_t launch_ggml_type(GemvArgs a, int nt, hipStream_t st) {
+  const int RB = 64 / (a.d >> 8);
+  const int want = ((a.n + RB - 1) / RB + 3) / 4;
+  const bool apart = want <= 3 * device_cus() || (T == kGgmlQ4 && nt <= 4);
+  if (nt > 1 && apart) return launch_ggml_t<T, 1>(a, st, nt);
   switch (nt) {
     case 1: return launch_ggml_t<T, 1>(a, st);
     case 2: return launch_ggml_t<T, 2>(a, st);
     case 3: return launch_ggml_t<T, 3>(a, st);
     case 4: return launch_ggml_t<T, 4>(a, st);
-    case 8: {
-      hipError_t e = launch_ggml_t<T, 4>(a, st);
-      if (e != hipSuccess) return e;
-      a.X += (size_t)4 * a.xstride;
-      a.Y += (size_t)4 * a.ystride;
-      return launch_ggml_t<T, 4>(a, st);
-    }
+    case 8: return launch_ggml_t<T, 4>(a, st, 2);
     default: return hipErrorInvalidValue;
   }
 }

@@ -372,6 +372,9 @@ void k_gemv_ggml(GemvArgs g) {
     g.W += (size_t)e * g.eslice;
     g.X += (size_t)(p / g.xk) * g.xstride;
     g.Y += (size_t)p * g.ystride;
+  } else {  // blockIdx.y: this workgroup row's NT tokens
+    g.X += (size_t)blockIdx.y * NT * g.xstride;
+    g.Y += (size_t)blockIdx.y * NT * g.ystride;
   }
   constexpr int BB = GgmlFmt<T>::kBytes, NDMA = GgmlFmt<T>::kDma;
   constexpr size_t SB = (size_t)NDMA * 1024;
