@@ -227,6 +227,9 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_gemv_blk(GemvArgs g) {
   const size_t tokb = act_tok_bytes(g.d);
   const int ntiles = (g.n + RB - 1) / RB;
   const int tstep = gridDim.x * kBlkWaves;
+  // blockIdx.y: this workgroup row's NT tokens
+  g.X += (size_t)blockIdx.y * NT * g.xstride;
+  g.Y += (size_t)blockIdx.y * NT * g.ystride;
   const size_t total = (size_t)g.n * rb;
   int tile = blockIdx.x * kBlkWaves + wave;
   const size_t tile_bytes = (size_t)RB * rb;
@@ -461,14 +464,41 @@ int resident_by_regs(const void* fn, int threads, std::atomic<int>& cache) {
 }
 
 template <int TYPE, int NT, bool XS, bool ACC>
-static hipError_t launch_blk_k(const GemvArgs& a, int grid, size_t lds, hipStream_t st) {
+static hipError_t launch_blk_k(const GemvArgs& a, int grid, size_t lds, hipStream_t st, int ny) {
   static std::atomic<bool> opted[64];
   if (lds > 64 * 1024) {
     hipError_t e = lds_opt_in((const void*)k_gemv_blk<TYPE, NT, XS, ACC>, opted);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_gemv_blk<TYPE, NT, XS, ACC>), dim3(grid), dim3(64 * kBlkWaves), lds, st, a);
+  hipLaunchKernelGGL((k_gemv_blk<TYPE, NT, XS, ACC>), dim3(grid, ny), dim3(64 * kBlkWaves), lds, st,
+                     a);
   return hipGetLastError();
+}
+
+// How many of a call's nt tokens share a workgroup; the rest are further rows
+// of workgroups (grid y) in the same launch, whose reads of the matrix the
+// caches serve.  Sharing saves decoding and LDS traffic, but it multiplies a
+// wave's serial work, so it pays only where the tiles fill the chip by
+// themselves: up to four tiles per CU (one per SIMD) the tokens go apart, by
+// twos where a token's tile work is long (Q5_K, Q6_K).  Measured, together and as
+// chosen, us: 5632 x 2048, four tokens, Q4_K tiled 7.8 -> 5.2 and row-major
+// 8.0 -> 5.6, Q5_K 8.2 -> 6.9, Q6_K 8.7 -> 8.0, Q8_0 7.7 -> 7.1 (three tokens
+// of Q6_K / Q8_0 apart: 7.3 -> 9.3, 6.6 -> 8.0, so they stay together); 2048 x
+// 5632, four tokens, 13.8 -> 9.9, 13.4 -> 10.6, 14.4 -> 11.6, 13.1 -> 9.6.  With
+// more tiles only Q4_K gains, in twos (32000 x 2048, four tokens: 14.1 -> 12.1;
+// Q5_K 16.3 -> 17.6, Q6_K 18.0 -> 21.3, Q8_0 18.3 -> 20.1, not taken).  Eight
+// tokens are one launch instead of two of four: 32000 x 2048 28.0 -> 19.4,
+// 32.5 -> 25.4, 36.0 -> 28.6, 36.5 -> 27.6.
+static int tokens_per_row(int type, bool tiled_k, int nt, int ntiles) {
+  const bool heavy = type == QR_T_Q5_K || type == QR_T_Q6_K;
+  const bool few = ntiles <= 4 * device_cus();
+  switch (nt) {
+    case 2: return few ? 1 : 2;
+    case 3: return few && (type == QR_T_Q4_K || (type == QR_T_Q5_K && tiled_k)) ? 1 : 3;
+    case 4: return few ? (heavy ? 2 : 1) : type == QR_T_Q4_K ? 2 : 4;
+    case 8: return few ? (heavy ? 2 : 1) : heavy ? 4 : 2;
+    default: return nt == 1 ? 1 : 0;  // 0: not a width of these kernels
+  }
 }
 
 // One tile in flight per wave and as many workgroups per CU as LDS holds, up
@@ -479,7 +509,7 @@ static hipError_t launch_blk_k(const GemvArgs& a, int grid, size_t lds, hipStrea
 // activation is staged through LDS by DMA when it fits kXsMax, else loaded
 // into registers (d = 5632 at 3 or 4 tokens).
 template <int TYPE, int NT>
-static hipError_t launch_blk_t(const GemvArgs& a, hipStream_t st) {
+static hipError_t launch_blk_t(const GemvArgs& a, hipStream_t st, int ny = 1) {
   const int nb = a.d >> 8;
   const int RB = 64 / nb;
   const bool xs = blk_xs_bytes(a.d, NT) <= kXsMax;
@@ -489,14 +519,14 @@ static hipError_t launch_blk_t(const GemvArgs& a, hipStream_t st) {
   const int want = (ntiles + kBlkWaves - 1) / kBlkWaves;
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 3 ? 3 : per_cu);
-  const int cap = device_cus() * per_cu;
+  const int cap = std::max(1, device_cus() * per_cu / ny);
   const int grid = want < cap ? want : cap;
   if (grid <= 0) return hipSuccess;
   const bool acc = a.acc || a.accb;
-  if (xs) return acc ? launch_blk_k<TYPE, NT, true, true>(a, grid, lds, st)
-                     : launch_blk_k<TYPE, NT, true, false>(a, grid, lds, st);
-  return acc ? launch_blk_k<TYPE, NT, false, true>(a, grid, lds, st)
-             : launch_blk_k<TYPE, NT, false, false>(a, grid, lds, st);
+  if (xs) return acc ? launch_blk_k<TYPE, NT, true, true>(a, grid, lds, st, ny)
+                     : launch_blk_k<TYPE, NT, true, false>(a, grid, lds, st, ny);
+  return acc ? launch_blk_k<TYPE, NT, false, true>(a, grid, lds, st, ny)
+             : launch_blk_k<TYPE, NT, false, false>(a, grid, lds, st, ny);
 }
 
 // The multi-token MFMA kernel (qr_gemv_mt.h); quads: the tokens as that many
@@ -530,19 +560,6 @@ static hipError_t launch_any_t(const GemvArgs& a, hipStream_t st) {
   if constexpr ((TYPE == QR_T_Q4_K || TYPE == QR_T_Q5_K) && NT <= 4) {
     if (gemv_blk_ok(TYPE, a.d, NT)) return launch_blk_t<TYPE, NT>(a, st);
   }
-  // Eight tokens as two passes of four: 32000 x 2048 Q4_K 28.5 us, 54.3 in the
-  // general kernel, whose every workgroup quantizes all eight tokens
-  // (256 x 768: 12.1 against 11.6).
-  if constexpr ((TYPE == QR_T_Q4_K || TYPE == QR_T_Q5_K) && NT == 8) {
-    if (!a.acc && !a.accb && gemv_blk_ok(TYPE, a.d, 4)) {
-      hipError_t e = launch_blk_t<TYPE, 4>(a, st);
-      if (e != hipSuccess) return e;
-      GemvArgs b = a;
-      b.X += (size_t)4 * a.xstride;
-      b.Y += (size_t)4 * a.ystride;
-      return launch_blk_t<TYPE, 4>(b, st);
-    }
-  }
   // Q6_K / Q8_0 of several tokens: the MFMA kernel (figures in qr_gemv_mt.h).
   // Two tokens of Q8_0 in the sequential order stay with the kernels below: the
   // streaming engine takes 20.1 us on 32000 x 2048 where this one takes 22.0.
@@ -567,6 +584,20 @@ static hipError_t launch_any_t(const GemvArgs& a, hipStream_t st) {
 
 template <int TYPE, int Q8O>
 static hipError_t launch_nt(const GemvArgs& a, int nt, hipStream_t st) {
+  if constexpr (TYPE == QR_T_Q4_K || TYPE == QR_T_Q5_K) {
+    // (the parity mode's integer sums: NT tokens per workgroup, below)
+    if (nt > 1 && !a.acc && !a.accb && gemv_blk_ok(TYPE, a.d, nt == 8 ? 4 : nt)) {
+      const int RB = 64 / (a.d >> 8);
+      const int m = tokens_per_row(TYPE, false, nt, (a.n + RB - 1) / RB);
+      switch (m) {
+        case 1: return launch_blk_t<TYPE, 1>(a, st, nt);
+        case 2: return launch_blk_t<TYPE, 2>(a, st, nt / 2);
+        case 3: return launch_blk_t<TYPE, 3>(a, st);
+        case 4: return launch_blk_t<TYPE, 4>(a, st, nt / 4);
+        default: return hipErrorInvalidValue;
+      }
+    }
+  }
   switch (nt) {
     case 1: return launch_any_t<TYPE, 1, Q8O>(a, st);
     case 2: return launch_any_t<TYPE, 2, Q8O>(a, st);
@@ -606,7 +637,7 @@ bool gemv_tiled_ok(int type, int n, int d, int nt, int q8o) {
 // workgroups per CU as the LDS holds (up to 4), the waves then walking their
 // tiles.
 template <int TYPE, int NT, int NW>
-static hipError_t launch_sq_nw(const GemvArgs& a, hipStream_t st) {
+static hipError_t launch_sq_nw(const GemvArgs& a, hipStream_t st, int ny) {
   static std::atomic<bool> opted[64];
   const SqGeom g = sq_geom(TYPE, a.n, a.d);
   if (g.ntiles <= 0) return hipSuccess;
@@ -618,53 +649,48 @@ static hipError_t launch_sq_nw(const GemvArgs& a, hipStream_t st) {
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
   const int want = (g.ntiles + NW - 1) / NW;
-  const int cap = device_cus() * per_cu;
+  const int cap = std::max(1, device_cus() * per_cu / ny);
   const int grid = want < cap ? want : cap;
-  hipLaunchKernelGGL((k_gemv_tiled_sq<TYPE, NT, NW>), dim3(grid), dim3(64 * NW), lds, st, a);
+  hipLaunchKernelGGL((k_gemv_tiled_sq<TYPE, NT, NW>), dim3(grid, ny), dim3(64 * NW), lds, st, a);
   return hipGetLastError();
 }
 template <int TYPE, int NT>
-static hipError_t launch_sq_t(const GemvArgs& a, hipStream_t st) {
-  if (sq_lds_bytes(TYPE, a.d, NT, 4) <= kLdsMax) return launch_sq_nw<TYPE, NT, 4>(a, st);
-  return launch_sq_nw<TYPE, NT, 2>(a, st);
+static hipError_t launch_sq_t(const GemvArgs& a, hipStream_t st, int ny = 1) {
+  if (sq_lds_bytes(TYPE, a.d, NT, 4) <= kLdsMax) return launch_sq_nw<TYPE, NT, 4>(a, st, ny);
+  return launch_sq_nw<TYPE, NT, 2>(a, st, ny);
 }
 
 template <int TYPE>
-static hipError_t launch_sq_type(GemvArgs a, int nt, hipStream_t st) {
-  switch (nt) {
-    case 1: return launch_sq_t<TYPE, 1>(a, st);
-    case 2: return launch_sq_t<TYPE, 2>(a, st);
+static hipError_t launch_sq_type(const GemvArgs& a, int nt, hipStream_t st) {
+  const int m = tokens_per_row(TYPE, false, nt, a.t_ntiles);
+  switch (m) {
+    case 1: return launch_sq_t<TYPE, 1>(a, st, nt);
+    case 2: return launch_sq_t<TYPE, 2>(a, st, nt / 2);
     case 3: return launch_sq_t<TYPE, 3>(a, st);
-    case 4: return launch_sq_t<TYPE, 4>(a, st);
-    case 8: {  // two launches of four tokens
-      hipError_t e = launch_sq_t<TYPE, 4>(a, st);
-      if (e != hipSuccess) return e;
-      a.X += (size_t)4 * a.xstride;
-      a.Y += (size_t)4 * a.ystride;
-      return launch_sq_t<TYPE, 4>(a, st);
-    }
+    case 4: return launch_sq_t<TYPE, 4>(a, st, nt / 4);
     default: return hipErrorInvalidValue;
   }
 }
 
 template <int TYPE, int NT, int NW, int PRO>
-static hipError_t launch_tiled_k(const GemvArgs& a, int grid, size_t lds, hipStream_t st) {
+static hipError_t launch_tiled_k(const GemvArgs& a, int grid, size_t lds, hipStream_t st,
+                                 int ny = 1) {
   static std::atomic<bool> opted[64];
   if (lds > 64 * 1024) {
     hipError_t e = lds_opt_in((const void*)k_gemv_tiled<TYPE, NT, NW, PRO>, opted);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_gemv_tiled<TYPE, NT, NW, PRO>), dim3(grid), dim3(64 * NW), lds, st, a);
+  hipLaunchKernelGGL((k_gemv_tiled<TYPE, NT, NW, PRO>), dim3(grid, ny), dim3(64 * NW), lds, st, a);
   return hipGetLastError();
 }
 
 template <int TYPE, int NT, int NW>
-static hipError_t launch_tiled_nw(const GemvArgs& a, int grid, size_t lds, hipStream_t st) {
+static hipError_t launch_tiled_nw(const GemvArgs& a, int grid, size_t lds, hipStream_t st, int ny) {
   constexpr int QW = NW < 4 ? NW : 4;
   const int groups = NT * (a.d >> 3);
-  if (groups <= 64 * QW) return launch_tiled_k<TYPE, NT, NW, kProAsm1>(a, grid, lds, st);
-  if (groups <= 128 * QW) return launch_tiled_k<TYPE, NT, NW, kProAsm2>(a, grid, lds, st);
-  return launch_tiled_k<TYPE, NT, NW, kProLate>(a, grid, lds, st);
+  if (groups <= 64 * QW) return launch_tiled_k<TYPE, NT, NW, kProAsm1>(a, grid, lds, st, ny);
+  if (groups <= 128 * QW) return launch_tiled_k<TYPE, NT, NW, kProAsm2>(a, grid, lds, st, ny);
+  return launch_tiled_k<TYPE, NT, NW, kProLate>(a, grid, lds, st, ny);
 }
 
 // Waves per workgroup: 8 where two such workgroups fit a CU's LDS and the
@@ -675,7 +701,7 @@ static hipError_t launch_tiled_nw(const GemvArgs& a, int grid, size_t lds, hipSt
 // wave one tile), 7.65 us; 4 waves, four per CU, 7.9 us; 16 waves, one per
 // CU, 8.3 us.
 template <int TYPE, int NT>
-static hipError_t launch_tiled_t(const GemvArgs& a, hipStream_t st) {
+static hipError_t launch_tiled_t(const GemvArgs& a, hipStream_t st, int ny = 1) {
   const TiledGeom g = tiled_geom(TYPE, a.n, a.d);
   if (g.ntiles <= 0) return hipSuccess;
   const int cus = device_cus();
@@ -685,25 +711,20 @@ static hipError_t launch_tiled_t(const GemvArgs& a, hipStream_t st) {
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
   const int want = (g.ntiles + nw - 1) / nw;
-  const int grid = want < cus * per_cu ? want : cus * per_cu;
-  if (nw == 8) return launch_tiled_nw<TYPE, NT, 8>(a, grid, lds, st);
-  return launch_tiled_nw<TYPE, NT, 4>(a, grid, lds, st);
+  const int cap = std::max(1, cus * per_cu / ny);
+  const int grid = want < cap ? want : cap;
+  if (nw == 8) return launch_tiled_nw<TYPE, NT, 8>(a, grid, lds, st, ny);
+  return launch_tiled_nw<TYPE, NT, 4>(a, grid, lds, st, ny);
 }
 
 template <int TYPE>
-static hipError_t launch_tiled_type(GemvArgs a, int nt, hipStream_t st) {
-  switch (nt) {
-    case 1: return launch_tiled_t<TYPE, 1>(a, st);
-    case 2: return launch_tiled_t<TYPE, 2>(a, st);
+static hipError_t launch_tiled_type(const GemvArgs& a, int nt, hipStream_t st) {
+  const int m = tokens_per_row(TYPE, true, nt, a.t_ntiles);
+  switch (m) {
+    case 1: return launch_tiled_t<TYPE, 1>(a, st, nt);
+    case 2: return launch_tiled_t<TYPE, 2>(a, st, nt / 2);
     case 3: return launch_tiled_t<TYPE, 3>(a, st);
-    case 4: return launch_tiled_t<TYPE, 4>(a, st);
-    case 8: {  // two launches of four tokens
-      hipError_t e = launch_tiled_t<TYPE, 4>(a, st);
-      if (e != hipSuccess) return e;
-      a.X += (size_t)4 * a.xstride;
-      a.Y += (size_t)4 * a.ystride;
-      return launch_tiled_t<TYPE, 4>(a, st);
-    }
+    case 4: return launch_tiled_t<TYPE, 4>(a, st, nt / 4);
     default: return hipErrorInvalidValue;
   }
 }

@@ -462,6 +462,9 @@ __device__ inline void tiled_body(const GemvArgs& g, uint8_t* smem, int bid, int
 template <int TYPE, int NT, int NW, int PRO>
 __global__ __launch_bounds__(64 * NW) void k_gemv_tiled(GemvArgs g) {
   extern __shared__ __align__(16) uint8_t smem[];
+  // blockIdx.y: this workgroup row's NT tokens
+  g.X += (size_t)blockIdx.y * NT * g.xstride;
+  g.Y += (size_t)blockIdx.y * NT * g.ystride;
   tiled_body<TYPE, NT, NW, PRO>(g, smem, (int)blockIdx.x, (int)gridDim.x);
 }
 
