@@ -916,50 +916,28 @@ __global__ __launch_bounds__(512) void k_attn_sv_rows(const float* __restrict__ 
   out[tid] = acc;
 }
 
-// The same attention values with the query heads of one kv head together:
-// workgroup (kv head blockIdx.x, token blockIdx.y) of kv_mul hd threads,
-// thread j hd + c = query head blockIdx.x kv_mul + j, column c.  Each head's softmax runs as in
-// k_attn_sv_rows (its max, exponentials, denominator by the head's first
-// thread, x *= inv); then the values in groups of kSgGrp positions: the
-// group's V values of the kv head are loaded into registers one group ahead,
-// dequantized into LDS once per workgroup, and every thread adds
-// e_j[t] * v[t][c] in position order -- the chains of k_attn_sv_rows, with
-// each V value read from L2 once per kv head instead of once per query head.
-// Dynamic LDS: kv_mul rows of ecap floats rounded up to 4 (the
-// exponentials), 2 x kSgGrp x hd
-// floats (the value tiles), ceil(ecap / page) ints (the page table).
-// kv_mul hd threads (a multiple of 64, at most 1024); NPER = kSgGrp / kv_mul
-// values per thread and group (kv_mul 4 or 8).
-constexpr int kSgGrp = 32;
-template <int KVT, int NPER>
-__global__ __launch_bounds__(1024) void k_attn_sv_gqa(const float* __restrict__ att,
-                                                     int att_stride, KvView V,
-                                                     const int32_t* __restrict__ st, int ecap,
-                                                     int kv_mul, int hd,
-                                                     float* __restrict__ out) {
+// Prefill, in two launches where a kv head serves four or eight query heads.
+//
+// k_softmax_chunk: softmax_ref (src/kernels.c:191-207) of each (token, head)'s
+// scores in place, a wave per row: the max (exact in any order), the
+// exponentials, their sum in position order (seq_sum_wave), x *= inv.  Bound by
+// the sums' chains.  grid (heads / RW, tokens), RW waves; dynamic LDS: RW rows of
+// ecap floats rounded up to 4.  The chunk's last token comes first: the longest
+// (causal) rows are dispatched first and the short ones fill in.
+__global__ __launch_bounds__(256) void k_softmax_chunk(float* __restrict__ att, int att_stride,
+                                                       const int32_t* __restrict__ st, int ecap,
+                                                       int nh) {
   extern __shared__ __align__(16) float sm[];
-  __shared__ float red[16];
-  __shared__ float inv_s[16];
-  const int tid = threadIdx.x, nthr = blockDim.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  // the chunk's last token first: its chains are the longest (causal), so
-  // the longest workgroups are dispatched first and the short ones fill in
-  const int kvh = blockIdx.x, z = gridDim.y - 1 - blockIdx.y;
-  const int nh = gridDim.x * kv_mul;
-  const int j = tid / hd, c = tid - j * hd;
-  const int h = kvh * kv_mul + j;
-  const int wph = hd >> 6;  // waves per head
-  const float* a = att + ((size_t)z * nh + h) * att_stride;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int z = gridDim.y - 1 - blockIdx.y;
+  const int h = blockIdx.x * (blockDim.x >> 6) + wave;
+  if (h >= nh) return;  // whole waves; no barriers
+  float* a = att + ((size_t)z * nh + h) * att_stride;
+  float* e = sm + (size_t)wave * ((ecap + 3) & ~3);
   const int npos = st[2 * z + 1] + 1;
-  const int es = (ecap + 3) & ~3;  // 16-byte aligned rows (float4 reads)
-  float* e = sm + (size_t)j * es;
-  float* vs = sm + (size_t)kv_mul * es;  // [2][kSgGrp][hd]
-  int32_t* pt = reinterpret_cast<int32_t*>(vs + 2 * kSgGrp * hd);
-  const int npg = (npos + V.page - 1) / V.page;
-  for (int i = tid; i < npg; i += nthr) pt[i] = V.ptab[i];
   const ExpTab tab = qr_expf_tab();
   float mx = a[0];
-  for (int i = c; i < npos; i += hd) {
+  for (int i = lane; i < npos; i += 64) {
     const float v = a[i];
     e[i] = v;
     mx = v > mx ? v : mx;
@@ -968,127 +946,225 @@ __global__ __launch_bounds__(1024) void k_attn_sv_gqa(const float* __restrict__ 
     const float v = __shfl_xor(mx, o);
     mx = v > mx ? v : mx;
   }
-  if (lane == 0) red[wave] = mx;
-  __syncthreads();
-  mx = red[j * wph];
-  for (int w = 1; w < wph; w++) mx = red[j * wph + w] > mx ? red[j * wph + w] : mx;
   // every lane runs the same number of rounds (qr_expf_w reads other lanes)
-  const int rounds = (npos + hd - 1) / hd;
-  for (int r = 0; r < rounds; r++) {
-    const int i = r * hd + c;
+  for (int i0 = 0; i0 < npos; i0 += 64) {
+    const int i = i0 + lane;
     const float v = i < npos ? e[i] : 0.0f;
     const float ev = qr_expf_w(v - mx, tab);
     if (i < npos) e[i] = ev;
   }
-  __syncthreads();
-  if (c == 0) inv_s[j] = 1.0f / seq_sum_lds_short(e, npos);
-  __syncthreads();
-  const float inv = inv_s[j];
-  for (int i = c; i < npos; i += hd) e[i] = e[i] * inv;  // softmax_ref's x[i] *= inv
-  // (the barrier of the first group below orders these writes before the adds)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the sum reads other lanes' terms
+  const float inv = 1.0f / seq_sum_wave<16>(e, npos, lane);
+  for (int i = lane; i < npos; i += 64) a[i] = e[i] * inv;
+}
 
-  // value k of a group: position g0 + (tid + nthr k) / hd, column (tid + nthr k) % hd
+// k_attn_values: o_h[c] = sum over t = 0 .. npos-1, in order, of p_h[t] * V[t][c]
+// for hd columns, the KM query heads of kv head blockIdx.x and TW tokens.  Thread
+// (token, group of HT heads, column c) carries HT chains of its column: V of
+// kSgGrp positions at a time is loaded into registers one group ahead, four columns
+// per load, and dequantized into LDS once for all of them; a value is read from
+// LDS once for HT chains; and the probabilities, the same for a whole wave, come
+// through scalar loads.  What bounds it: the multiplies and adds (VALU, 27 us at 512
+// tokens of 32 heads, head_dim 128) and, beside them, the scalar loads' latency
+// and the staging.  45 us there, with 17 us for the softmax; one launch of a
+// workgroup of kv_mul hd threads per token, one chain per thread, was bound by its
+// LDS reads (two for each multiply-add) and took 118.  V staged one value per
+// load, with eight heads per thread: 72 us.
+// grid (kv heads, token groups): the first half of the groups from the chunk's
+// end down, then the rest from its start up, so that the workgroups sharing a CU
+// have short and long chains between them.  Dynamic LDS: 2 x kSgGrp x hd floats
+// (the value tiles), ceil(ecap / page) ints (the page table).  NPER = kSgGrp hd /
+// threads values staged per thread and group.
+constexpr int kSgGrp = 32;
+constexpr int kAvThreads = 512;
+template <int KVT, int KM, int HT, int NPER>
+__global__ __launch_bounds__(kAvThreads) void k_attn_values(const float* __restrict__ att,
+                                                            int att_stride, KvView V,
+                                                            const int32_t* __restrict__ st,
+                                                            int hd, int tokens,
+                                                            float* __restrict__ out) {
+  extern __shared__ __align__(16) float sm[];
+  float* vs = sm;  // [2][kSgGrp][hd]
+  typedef const __attribute__((address_space(4))) float CFloat;
+  const int tid = threadIdx.x, nthr = blockDim.x;
+  constexpr int HG = KM / HT;  // waves' head groups
+  const int TW = nthr / (hd * HG);
+  const int ng = gridDim.y, half = (ng + 1) / 2, y = blockIdx.y;
+  const int z0 = (y < half ? ng - 1 - y : y - half) * TW;
+  const int kvh = blockIdx.x, nh = gridDim.x * KM;
+  // a wave is whole in one token (hd is a multiple of 64)
+  const int col = __builtin_amdgcn_readfirstlane(tid / hd), c = tid - col * hd;
+  const int tl = col / HG, j0 = (col - tl * HG) * HT;
+  const int z = min(z0 + tl, tokens - 1);
+  const bool live = z0 + tl < tokens;
+  const int npos = live ? st[2 * z + 1] + 1 : 0;
+  int nmax = 0;
+  for (int i = 0; i < TW; i++) nmax = max(nmax, st[2 * min(z0 + i, tokens - 1) + 1] + 1);
+  int32_t* pt = reinterpret_cast<int32_t*>(vs + 2 * kSgGrp * hd);
+  const int npg = (nmax + V.page - 1) / V.page;
+  for (int i = tid; i < npg; i += nthr) pt[i] = V.ptab[i];
+  CFloat* pr = (CFloat*)(att + ((size_t)z * nh + (size_t)kvh * KM + j0) * att_stride);
+
+  // quad k of a group: position g0 + q / hd4, columns 4 (q % hd4) .. + 3 with
+  // q = tid + nthr k, so that a row's address and a block's scale serve four values
   const size_t col0 = (size_t)kvh * hd;
-  uint32_t rq[NPER], rd[NPER];
+  constexpr int NQ = NPER / 4, NW = KVT == QR_KV_F32 ? 4 : KVT == QR_KV_F16 ? 2 : 1;
+  typedef uint32_t u32a2 __attribute__((aligned(2)));
+  uint32_t rq[NQ][NW], rd[NQ];
   auto load = [&](int g0) {
 #pragma unroll
-    for (int k = 0; k < NPER; k++) {
-      const int idx = tid + nthr * k;
-      const int u = idx / hd, cc = idx - u * hd;
-      const int t = min(g0 + u, npos - 1);  // past the end: reload the last row
+    for (int k = 0; k < NQ; k++) {
+      const int q = tid + nthr * k, hd4 = hd >> 2;
+      const int u = q / hd4, cc = 4 * (q - u * hd4);
+      const int t = min(g0 + u, nmax - 1);  // past the end: reload the last row
       const uint8_t* row = kv_row_lds(V, pt, t);
       if constexpr (KVT == QR_KV_Q8_0) {
         const uint8_t* blk = row + ((col0 + cc) >> 5) * QR_Q8_BYTES;
         rd[k] = *reinterpret_cast<const uint16_t*>(blk);
-        rq[k] = (uint32_t)blk[2 + ((col0 + cc) & 31)];
+        rq[k][0] = *reinterpret_cast<const u32a2*>(blk + 2 + ((col0 + cc) & 31));
       } else if constexpr (KVT == QR_KV_F16) {
-        rq[k] = reinterpret_cast<const uint16_t*>(row)[col0 + cc];
+        const uint2 w = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(row) + col0 + cc);
+        rq[k][0] = w.x;
+        rq[k][1] = w.y;
       } else {
-        rq[k] = reinterpret_cast<const uint32_t*>(row)[col0 + cc];
+        const uint4 w = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint32_t*>(row) + col0 + cc);
+        rq[k][0] = w.x;
+        rq[k][1] = w.y;
+        rq[k][2] = w.z;
+        rq[k][3] = w.w;
       }
     }
   };
   __syncthreads();  // the page table
   load(0);
-  float acc = 0.0f;
+  float acc[HT];
+#pragma unroll
+  for (int j = 0; j < HT; j++) acc[j] = 0.0f;
   int buf = 0;
-  for (int g0 = 0; g0 < npos; g0 += kSgGrp) {
+  for (int g0 = 0; g0 < nmax; g0 += kSgGrp) {
     float* vb = vs + buf * kSgGrp * hd;
 #pragma unroll
-    for (int k = 0; k < NPER; k++) {
-      const int idx = tid + nthr * k;
-      float v;
-      if constexpr (KVT == QR_KV_Q8_0) v = (float)(int8_t)(uint8_t)rq[k] * qr_h2f((uint16_t)rd[k]);
-      else if constexpr (KVT == QR_KV_F16) v = qr_h2f(rq[k]);
-      else v = __uint_as_float(rq[k]);
-      vb[idx] = v;  // [u][cc] = idx
+    for (int k = 0; k < NQ; k++) {
+      float4 v;
+      if constexpr (KVT == QR_KV_Q8_0) {
+        const float d = qr_h2f((uint16_t)rd[k]);
+        const uint32_t w = rq[k][0];
+        v = make_float4((float)(int8_t)w * d, (float)(int8_t)(w >> 8) * d, (float)(int8_t)(w >> 16) * d,
+                        (float)(int8_t)(w >> 24) * d);
+      } else if constexpr (KVT == QR_KV_F16) {
+        v = make_float4(qr_h2f(rq[k][0] & 0xFFFFu), qr_h2f(rq[k][0] >> 16),
+                        qr_h2f(rq[k][1] & 0xFFFFu), qr_h2f(rq[k][1] >> 16));
+      } else {
+        v = make_float4(__uint_as_float(rq[k][0]), __uint_as_float(rq[k][1]),
+                        __uint_as_float(rq[k][2]), __uint_as_float(rq[k][3]));
+      }
+      *reinterpret_cast<float4*>(vb + 4 * (tid + nthr * k)) = v;  // [u][cc]
     }
     __syncthreads();
-    if (g0 + kSgGrp < npos) load(g0 + kSgGrp);
-    const int n = min(kSgGrp, npos - g0);
+    if (g0 + kSgGrp < nmax) load(g0 + kSgGrp);
+    const int n = min(kSgGrp, npos - g0);  // uniform in a wave
     if (n == kSgGrp) {
+#pragma unroll 2
+      for (int u = 0; u < kSgGrp; u += 4) {
+        float p[HT][4], v[4];
 #pragma unroll
-      for (int u = 0; u < kSgGrp; u++) acc += e[g0 + u] * vb[u * hd + c];
+        for (int i = 0; i < 4; i++) v[i] = vb[(u + i) * hd + c];
+#pragma unroll
+        for (int j = 0; j < HT; j++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) p[j][i] = pr[(size_t)j * att_stride + g0 + u + i];
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < HT; j++) acc[j] += p[j][i] * v[i];
+      }
     } else {
-      for (int u = 0; u < n; u++) acc += e[g0 + u] * vb[u * hd + c];
+      for (int u = 0; u < n; u++) {
+        const float v = vb[u * hd + c];
+#pragma unroll
+        for (int j = 0; j < HT; j++) acc[j] += pr[(size_t)j * att_stride + g0 + u] * v;
+      }
     }
     buf ^= 1;
   }
-  out[((size_t)z * nh + h) * hd + c] = acc;
+  if (live)
+#pragma unroll
+    for (int j = 0; j < HT; j++) out[((size_t)z * nh + kvh * KM + j0 + j) * hd + c] = acc[j];
 }
 
-// Whether k_attn_sv_gqa takes a chunk whose positions stop below ecap.
-inline size_t sv_gqa_lds(int ecap, int kv_mul, int hd, int page) {
-  return ((size_t)kv_mul * ((ecap + 3) & ~3) + 2 * (size_t)kSgGrp * hd) * 4 +
-         (size_t)((ecap + page - 1) / page) * 4;
+// Whether the two launches take a chunk whose positions stop below ecap: rows
+// of the softmax in 64 KiB of LDS (4 waves a workgroup, 2 or 1 for long rows).
+inline int softmax_rows(int ecap) { return ecap <= 4096 ? 4 : ecap <= 8192 ? 2 : 1; }
+inline bool attn_values_ok(int ecap, int kv_mul, int hd) {
+  return (kv_mul == 4 || kv_mul == 8) && hd % 64 == 0 && hd <= 256 && ecap >= 1 && ecap <= 16384;
 }
-// k_attn_sv_gqa's static LDS (red[16] and inv_s[16]): the dynamic part may
-// take only what it leaves of the CU's 160 KiB.
-constexpr size_t kSvGqaStatic = 2 * 16 * sizeof(float);
-inline bool sv_gqa_ok(int ecap, int kv_mul, int hd, int page) {
-  // kv_mul 1 and 2 (16 and 32 values per thread and group) would spill
-  return (kv_mul == 4 || kv_mul == 8) && hd % 64 == 0 && kv_mul * hd <= 1024 && ecap >= 1 &&
-         sv_gqa_lds(ecap, kv_mul, hd, page) + kSvGqaStatic <= kDecLdsMax;
-}
-template <int KVT, int NPER>
-std::atomic<bool>* gqa_opt() {
+template <int KVT, int KM, int HT, int NPER>
+hipError_t values_launch_n(const float* att, int att_stride, const KvView& V, const int32_t* st,
+                           int ecap, int nkv, int hd, float* out, int tokens, hipStream_t s) {
   static std::atomic<bool> f[64];
-  return f;
-}
-template <int KVT, int NPER>
-hipError_t gqa_launch(dim3 g, int threads, size_t lds, hipStream_t s, const float* att,
-                      int att_stride, const KvView& V, const int32_t* st, int ecap, int kv_mul,
-                      int hd, float* out) {
+  const int TW = kSgGrp / NPER * HT / KM;
+  const size_t lds = 2 * (size_t)kSgGrp * hd * 4 + (size_t)((ecap + V.page - 1) / V.page) * 4;
   if (lds > 64 * 1024) {
-    const hipError_t e = lds_opt_in((const void*)k_attn_sv_gqa<KVT, NPER>, gqa_opt<KVT, NPER>());
+    const hipError_t e = lds_opt_in((const void*)k_attn_values<KVT, KM, HT, NPER>, f);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((k_attn_sv_gqa<KVT, NPER>), g, dim3(threads), lds, s, att, att_stride, V, st,
-                     ecap, kv_mul, hd, out);
+  hipLaunchKernelGGL((k_attn_values<KVT, KM, HT, NPER>), dim3(nkv, (tokens + TW - 1) / TW),
+                     dim3(TW * (KM / HT) * hd), lds, s, att, att_stride, V, st, hd, tokens, out);
   return hipGetLastError();
 }
+template <int KVT, int KM, int HT>
+hipError_t values_launch_h(const float* att, int att_stride, const KvView& V, const int32_t* st,
+                           int ecap, int nkv, int hd, float* out, int tokens, hipStream_t s) {
+  const int cols = kAvThreads / hd;  // (token, head group)s of a workgroup: 8, 4, 2
+  if (cols == 8)
+    return values_launch_n<KVT, KM, HT, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if (cols == 4)
+    return values_launch_n<KVT, KM, HT, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if constexpr (KM / HT <= 2)
+    return values_launch_n<KVT, KM, HT, 16>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  return hipErrorInvalidValue;  // not chosen below
+}
+template <int KVT, int KM>
+hipError_t values_launch(const float* att, int att_stride, const KvView& V, const int32_t* st,
+                         int ecap, int nkv, int hd, float* out, int tokens, hipStream_t s) {
+  // Four heads per thread where that leaves four waves on each SIMD, else two:
+  // 512-token prompt (4 layers, 8:1, head_dim 128) 2113 us with four, 2152 with
+  // two, 2213 with eight; 300 tokens (8:1, head_dim 64) 1293, 1271 and 1360.
+  if constexpr (KM == 8) {
+    const bool wide = 2L * tokens * nkv * (hd / 64) >= 16L * device_cus();
+    if (wide || kAvThreads / hd < 4)
+      return values_launch_h<KVT, KM, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  }
+  return values_launch_h<KVT, KM, 2>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+}
 template <int KVT>
-hipError_t gqa_launch_kv(dim3 g, size_t lds, hipStream_t s, const float* att, int att_stride,
-                         const KvView& V, const int32_t* st, int ecap, int kv_mul, int hd,
-                         float* out) {
-  const int threads = kv_mul * hd;
-  if (kv_mul == 8)
-    return gqa_launch<KVT, 4>(g, threads, lds, s, att, att_stride, V, st, ecap, kv_mul, hd, out);
-  return gqa_launch<KVT, 8>(g, threads, lds, s, att, att_stride, V, st, ecap, kv_mul, hd, out);
+hipError_t values_launch_kv(const float* att, int att_stride, const KvView& V, const int32_t* st,
+                            int ecap, int nkv, int kv_mul, int hd, float* out, int tokens,
+                            hipStream_t s) {
+  return kv_mul == 8
+             ? values_launch<KVT, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s)
+             : values_launch<KVT, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
 }
 
 // ecap: the chunk's positions end (every token's npos <= ecap).
-hipError_t sv_rows_launch(const float* att, int att_stride, const KvView& V, const int32_t* st,
+// The scores become probabilities in place where the two launches take them.
+hipError_t sv_rows_launch(float* att, int att_stride, const KvView& V, const int32_t* st,
                           int lds_cap, int n_heads, int kv_mul, int hd, float* out, int tokens,
                           hipStream_t s, int ecap = 0) {
-  if (ecap > 0 && sv_gqa_ok(ecap, kv_mul, hd, V.page)) {
-    const dim3 g(n_heads / kv_mul, tokens);
-    const size_t l = sv_gqa_lds(ecap, kv_mul, hd, V.page);
+  if (ecap > 0 && attn_values_ok(ecap, kv_mul, hd)) {
+    const int rw = softmax_rows(ecap);
+    hipLaunchKernelGGL(k_softmax_chunk, dim3((n_heads + rw - 1) / rw, tokens), dim3(64 * rw),
+                       (size_t)rw * ((ecap + 3) & ~3) * 4, s, att, att_stride, st, ecap, n_heads);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const int nkv = n_heads / kv_mul;
     if (V.kv_type == QR_KV_Q8_0)
-      return gqa_launch_kv<QR_KV_Q8_0>(g, l, s, att, att_stride, V, st, ecap, kv_mul, hd, out);
+      return values_launch_kv<QR_KV_Q8_0>(att, att_stride, V, st, ecap, nkv, kv_mul, hd, out,
+                                          tokens, s);
     if (V.kv_type == QR_KV_F16)
-      return gqa_launch_kv<QR_KV_F16>(g, l, s, att, att_stride, V, st, ecap, kv_mul, hd, out);
-    return gqa_launch_kv<QR_KV_F32>(g, l, s, att, att_stride, V, st, ecap, kv_mul, hd, out);
+      return values_launch_kv<QR_KV_F16>(att, att_stride, V, st, ecap, nkv, kv_mul, hd, out, tokens,
+                                         s);
+    return values_launch_kv<QR_KV_F32>(att, att_stride, V, st, ecap, nkv, kv_mul, hd, out, tokens, s);
   }
   const dim3 grid(n_heads, tokens);
   const int threads = ((hd + 63) / 64) * 64;
