@@ -432,7 +432,37 @@ __global__ __launch_bounds__(256) void k_attn_scores(const float* __restrict__ q
     }
     *reinterpret_cast<float4*>(qs + i) = a;
   }
-  if (ROPE && cur >= 0 && cur < kScTile && (int)threadIdx.x < 2 * (hd / 32)) {
+  if (ROPE && K.kv_type != QR_KV_Q8_0 && cur >= 0 && cur < kScTile && (int)threadIdx.x < hd / 2) {
+    // fp16 / fp32 rows: four values of kv head kvh's k (rotated) or v per thread.
+    // (A thread per block of 32 ran its 64 fp16 conversions, with their range
+    // branches, one after the other: 8-layer decode step over 702 fp16
+    // positions, head_dim 64, 596 us; 569 so.)
+    const bool isv = (int)threadIdx.x >= hd / 4;
+    const int i = 4 * ((int)threadIdx.x - (isv ? hd / 4 : 0));
+    const size_t e = (size_t)kvh * hd + i;
+    float4 f = *reinterpret_cast<const float4*>((isv ? R.v : R.k) + e);
+    if (!isv) {
+      const float4 c = *reinterpret_cast<const float4*>(cs + e);
+      const float4 r = f;
+      f.x = r.x * c.x - r.y * c.y;
+      f.y = r.x * c.y + r.y * c.x;
+      f.z = r.z * c.z - r.w * c.w;
+      f.w = r.z * c.w + r.w * c.z;
+    }
+    uint8_t* krow = const_cast<uint8_t*>(K.row(npos - 1));
+    uint8_t* row = isv ? R.vbase + (size_t)(krow - K.base) : krow;
+    if (K.kv_type == QR_KV_F16) {
+      const uint32_t h0 = qr_f2h(f.x), h1 = qr_f2h(f.y), h2 = qr_f2h(f.z), h3 = qr_f2h(f.w);
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(row) + e) =
+          make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+      f = make_float4(qr_h2f(h0), qr_h2f(h1), qr_h2f(h2), qr_h2f(h3));  // as the cache holds it
+    } else {
+      *reinterpret_cast<float4*>(reinterpret_cast<float*>(row) + e) = f;
+    }
+    if (!isv) *reinterpret_cast<float4*>(kt + cur * ks + i) = f;
+  }
+  if (ROPE && K.kv_type == QR_KV_Q8_0 && cur >= 0 && cur < kScTile &&
+      (int)threadIdx.x < 2 * (hd / 32)) {
     // block b of kv head kvh's k (rotated) or v, at the current position
     const int nbh = hd / 32;
     const bool isv = (int)threadIdx.x >= nbh;
@@ -463,27 +493,12 @@ __global__ __launch_bounds__(256) void k_attn_scores(const float* __restrict__ q
     uint8_t* krow = const_cast<uint8_t*>(K.row(npos - 1));
     uint8_t* row = isv ? R.vbase + (size_t)(krow - K.base) : krow;
     float* dst = kt + cur * ks + 32 * b;
-    if (K.kv_type == QR_KV_Q8_0) {
-      uint8_t* blk = row + (size_t)(kvh * nbh + b) * QR_Q8_BYTES;
-      q8_block_store(vals, blk);
-      if (!isv) {  // the row as the cache holds it
-        const float d = qr_h2f((uint32_t)blk[0] | ((uint32_t)blk[1] << 8));
+    uint8_t* blk = row + (size_t)(kvh * nbh + b) * QR_Q8_BYTES;
+    q8_block_store(vals, blk);
+    if (!isv) {  // the row as the cache holds it
+      const float d = qr_h2f((uint32_t)blk[0] | ((uint32_t)blk[1] << 8));
 #pragma unroll
-        for (int j = 0; j < 32; j++) dst[j] = (float)(int8_t)blk[2 + j] * d;
-      }
-    } else if (K.kv_type == QR_KV_F16) {
-      f16_block_store(vals, row + (size_t)(kvh * nbh + b) * 64);
-      if (!isv) {
-#pragma unroll
-        for (int j = 0; j < 32; j++) dst[j] = qr_h2f(qr_f2h(vals[j]));
-      }
-    } else {
-      float* out = reinterpret_cast<float*>(row) + (size_t)kvh * hd + 32 * b;
-#pragma unroll
-      for (int j = 0; j < 32; j++) {
-        out[j] = vals[j];
-        if (!isv) dst[j] = vals[j];
-      }
+      for (int j = 0; j < 32; j++) dst[j] = (float)(int8_t)blk[2 + j] * d;
     }
   }
   if (K.kv_type == QR_KV_Q8_0) {

@@ -228,8 +228,10 @@ __global__ __launch_bounds__(64 * kBlkWaves) void k_gemv_blk(GemvArgs g) {
   const int ntiles = (g.n + RB - 1) / RB;
   const int tstep = gridDim.x * kBlkWaves;
   // blockIdx.y: this workgroup row's NT tokens
-  g.X += (size_t)blockIdx.y * NT * g.xstride;
-  g.Y += (size_t)blockIdx.y * NT * g.ystride;
+  if (blockIdx.y) {
+    g.X += (size_t)blockIdx.y * NT * g.xstride;
+    g.Y += (size_t)blockIdx.y * NT * g.ystride;
+  }
   const size_t total = (size_t)g.n * rb;
   int tile = blockIdx.x * kBlkWaves + wave;
   const size_t tile_bytes = (size_t)RB * rb;

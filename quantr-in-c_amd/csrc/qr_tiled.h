@@ -463,8 +463,10 @@ template <int TYPE, int NT, int NW, int PRO>
 __global__ __launch_bounds__(64 * NW) void k_gemv_tiled(GemvArgs g) {
   extern __shared__ __align__(16) uint8_t smem[];
   // blockIdx.y: this workgroup row's NT tokens
-  g.X += (size_t)blockIdx.y * NT * g.xstride;
-  g.Y += (size_t)blockIdx.y * NT * g.ystride;
+  if (blockIdx.y) {
+    g.X += (size_t)blockIdx.y * NT * g.xstride;
+    g.Y += (size_t)blockIdx.y * NT * g.ystride;
+  }
   tiled_body<TYPE, NT, NW, PRO>(g, smem, (int)blockIdx.x, (int)gridDim.x);
 }
 
