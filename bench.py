@@ -838,7 +838,10 @@ def main():
 
     cpus = host_cpus()
     cpu = None
-    if not args.no_cpu:
+    have_ref = os.path.exists(os.path.join(REPO, "oracle", "_ref", "libqref_avx2.so"))
+    if not args.no_cpu and not have_ref:
+        log("bench: no CPU baseline: the reference's sources were not here to build oracle/_ref")
+    if not args.no_cpu and have_ref:
         cpu = cpu_baseline_gemv(cpus)
         if M is not None:
             moe["cpu_baseline"] = cpu_baseline_moe(M, cpus)
