@@ -931,7 +931,8 @@ __global__ __launch_bounds__(512) void k_attn_sv_rows(const float* __restrict__ 
   out[tid] = acc;
 }
 
-// Prefill, in two launches where a kv head serves four or eight query heads.
+// Prefill, in two launches where a kv head serves four or eight query heads and the
+// chunk is not short (values_two_launches below).
 //
 // k_softmax_chunk: softmax_ref (src/kernels.c:191-207) of each (token, head)'s
 // scores in place, a wave per row: the max (exact in any order), the
@@ -1127,38 +1128,81 @@ hipError_t values_launch_n(const float* att, int att_stride, const KvView& V, co
                      dim3(TW * (KM / HT) * hd), lds, s, att, att_stride, V, st, hd, tokens, out);
   return hipGetLastError();
 }
-template <int KVT, int KM, int HT>
-hipError_t values_launch_h(const float* att, int att_stride, const KvView& V, const int32_t* st,
-                           int ecap, int nkv, int hd, float* out, int tokens, hipStream_t s) {
+// Query heads per thread of k_attn_values.  One where the kv head's heads then
+// still fit a workgroup and its workgroups number at most two per CU: few tokens
+// leave the chip idle, and more workgroups of shorter work fill it (2-layer prompts,
+// 8:1, head_dim 64: 24 tokens at position 2000 of an fp16 cache 659 us with two
+// heads per thread, 592 with one; 64 tokens at 4000, Q8_0, 897 and 838; 300 tokens
+// there 1942 and 2061).  Four where that leaves four waves on each SIMD, or where two
+// do not fit, else two: 512-token prompt (4 layers, 8:1, head_dim 128) 2113 us with
+// four, 2152 with two, 2213 with eight; 300 tokens (8:1, head_dim 64) 1293, 1271
+// and 1360.
+inline int values_heads(int kv_type, int tokens, int nkv, int kv_mul, int hd) {
   const int cols = kAvThreads / hd;  // (token, head group)s of a workgroup: 8, 4, 2
-  if (cols == 8)
-    return values_launch_n<KVT, KM, HT, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
-  if (cols == 4)
-    return values_launch_n<KVT, KM, HT, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
-  if constexpr (KM / HT <= 2)
-    return values_launch_n<KVT, KM, HT, 16>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
-  return hipErrorInvalidValue;  // not chosen below
-}
-template <int KVT, int KM>
-hipError_t values_launch(const float* att, int att_stride, const KvView& V, const int32_t* st,
-                         int ecap, int nkv, int hd, float* out, int tokens, hipStream_t s) {
-  // Four heads per thread where that leaves four waves on each SIMD, else two:
-  // 512-token prompt (4 layers, 8:1, head_dim 128) 2113 us with four, 2152 with
-  // two, 2213 with eight; 300 tokens (8:1, head_dim 64) 1293, 1271 and 1360.
-  if constexpr (KM == 8) {
-    const bool wide = 2L * tokens * nkv * (hd / 64) >= 16L * device_cus();
-    if (wide || kAvThreads / hd < 4)
-      return values_launch_h<KVT, KM, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if (kv_type != QR_KV_F32 && cols >= kv_mul) {
+    const int tw = cols / kv_mul;
+    if ((long)nkv * ((tokens + tw - 1) / tw) <= 2L * device_cus()) return 1;
   }
-  return values_launch_h<KVT, KM, 2>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if (kv_mul == 8 && (cols < 4 || 2L * tokens * nkv * (hd / 64) >= 16L * device_cus())) return 4;
+  return 2;
+}
+
+// Whether the two launches beat one workgroup per (head, token)
+// (k_attn_sv_rows), which has kv_mul times their workgroups and reads V that often.
+// With one head per thread they do.  With more, beyond one workgroup for four CUs
+// (2-layer prompts, 8:1, us with two launches and per head: head_dim 128, 16 tokens
+// at position 9000, fp16, 1880 and 1604, at 4000 1001 and 961, 24 tokens 1171 and 1186;
+// head_dim 256, fp16, position 4000, 16 tokens 1070 and 756, 32 tokens 1151 and 959, 64
+// tokens 1294 and 1411).  fp32 rows need no conversion, so that sharing one pays
+// only beyond two (token, kv head)s per CU (8:1, head_dim 64, position 4000: 24 tokens 929
+// and 624, 64 tokens 881 and 700, 160 tokens 1370 and 1409).
+inline bool values_two_launches(int kv_type, int tokens, int nkv, int kv_mul, int hd) {
+  if (kv_type == QR_KV_F32) return (long)nkv * tokens > 2L * device_cus();
+  const int ht = values_heads(kv_type, tokens, nkv, kv_mul, hd);
+  if (ht == 1) return true;
+  const int tw = kAvThreads / hd * ht / kv_mul;
+  return (long)nkv * ((tokens + tw - 1) / tw) > device_cus() / 4;
+}
+
+// ht: values_heads above
+template <int KVT, int KM>
+hipError_t values_launch(int ht, const float* att, int att_stride, const KvView& V,
+                         const int32_t* st, int ecap, int nkv, int hd, float* out, int tokens,
+                         hipStream_t s) {
+  const int cols = kAvThreads / hd;
+  if constexpr (KVT != QR_KV_F32) {
+    if (ht == 1 && cols == 8)
+      return values_launch_n<KVT, KM, 1, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+    if constexpr (KM == 4) {
+      if (ht == 1 && cols == 4)
+        return values_launch_n<KVT, KM, 1, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+    }
+  }
+  if (ht == 2 && cols == 8)
+    return values_launch_n<KVT, KM, 2, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if (ht == 2 && cols == 4)
+    return values_launch_n<KVT, KM, 2, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  if constexpr (KM == 4) {
+    if (ht == 2 && cols == 2)
+      return values_launch_n<KVT, KM, 2, 16>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  } else {
+    if (ht == 4 && cols == 8)
+      return values_launch_n<KVT, KM, 4, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+    if (ht == 4 && cols == 4)
+      return values_launch_n<KVT, KM, 4, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+    if (ht == 4 && cols == 2)
+      return values_launch_n<KVT, KM, 4, 16>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+  }
+  return hipErrorInvalidValue;  // not chosen by values_heads
 }
 template <int KVT>
 hipError_t values_launch_kv(const float* att, int att_stride, const KvView& V, const int32_t* st,
                             int ecap, int nkv, int kv_mul, int hd, float* out, int tokens,
                             hipStream_t s) {
+  const int ht = values_heads(KVT, tokens, nkv, kv_mul, hd);
   return kv_mul == 8
-             ? values_launch<KVT, 8>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s)
-             : values_launch<KVT, 4>(att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
+             ? values_launch<KVT, 8>(ht, att, att_stride, V, st, ecap, nkv, hd, out, tokens, s)
+             : values_launch<KVT, 4>(ht, att, att_stride, V, st, ecap, nkv, hd, out, tokens, s);
 }
 
 // ecap: the chunk's positions end (every token's npos <= ecap).
@@ -1166,7 +1210,8 @@ hipError_t values_launch_kv(const float* att, int att_stride, const KvView& V, c
 hipError_t sv_rows_launch(float* att, int att_stride, const KvView& V, const int32_t* st,
                           int lds_cap, int n_heads, int kv_mul, int hd, float* out, int tokens,
                           hipStream_t s, int ecap = 0) {
-  if (ecap > 0 && attn_values_ok(ecap, kv_mul, hd)) {
+  if (ecap > 0 && attn_values_ok(ecap, kv_mul, hd) &&
+      values_two_launches(V.kv_type, tokens, n_heads / kv_mul, kv_mul, hd)) {
     const int rw = softmax_rows(ecap);
     hipLaunchKernelGGL(k_softmax_chunk, dim3((n_heads + rw - 1) / rw, tokens), dim3(64 * rw),
                        (size_t)rw * ((ecap + 3) & ~3) * 4, s, att, att_stride, st, ecap, n_heads);
@@ -1183,6 +1228,9 @@ hipError_t sv_rows_launch(float* att, int att_stride, const KvView& V, const int
   }
   const dim3 grid(n_heads, tokens);
   const int threads = ((hd + 63) / 64) * 64;
+  // LDS for the positions there are: the whole capacity of a long cache would
+  // leave one workgroup on a CU
+  if (ecap > 0) lds_cap = std::min(lds_cap, (ecap + 63) & ~63);
   const size_t lds = (size_t)lds_cap * 4;
   if (V.kv_type == QR_KV_Q8_0)
     hipLaunchKernelGGL(k_attn_sv_rows<QR_KV_Q8_0>, grid, dim3(threads), lds, s, att, att_stride, V,

@@ -175,12 +175,11 @@ def test_prefill_gqa8_chunks(dev, oracle, kv_type, page):
 
 
 def test_prefill_gqa8_lds_boundary(dev, oracle):
-    """GQA 8:1 at head_dim 128 in pages of 256 near 4096 positions, where the
-    per-kv-head values kernel's LDS (eight score rows of the chunk's extent
-    plus the value tiles and page table) reaches the CU's 160 KiB: a chunk
-    ending at extent 4088 still fits it, one ending at 4092 runs the per-head
-    kernel instead.  The prefix is prefilled on the device; the oracle then
-    runs the two chunks' tokens over that cache: every logit bit-exact."""
+    """GQA 8:1 at head_dim 128 in pages of 256 near 4096 positions: chunks of eight
+    and four tokens (each head and token its own workgroup, LDS for the chunk's
+    extent: 4088 and 4092).  The prefix is prefilled on the device; the oracle then
+    runs the two chunks' tokens over that cache: every logit bit-exact.  (The
+    lines between the routes: test_gpu_prefill_routes.py.)"""
     m = I.qwen3_small_model(n_layers=1, seq_len=4096, n_kv_heads=1)
     rng = np.random.default_rng(41)
     toks = rng.integers(0, m["vocab"], size=4092).astype(np.int32)

@@ -1,8 +1,8 @@
-"""The prefill attention's softmax and value launches at the edges of their
-split: token groups that do not divide the chunk, position groups of 32 cut
-short, both head-group widths (few and many tokens), each cache type and pages
-smaller than a position group.  Bit-exact with the oracle's token-by-token
-decode.
+"""The prefill attention at the edges of its split: token groups that do not
+divide the chunk, position groups of 32 cut short, few tokens (a workgroup per
+head and token, or one head per thread) and many (four heads per thread), each
+cache type and pages smaller than a position group.  Bit-exact with the oracle's
+token-by-token decode.
 """
 import numpy as np
 import pytest

@@ -11,12 +11,9 @@ every layer runs the same kernels, and the oracle's cost grows with each.
 - Three decode steps at positions 4096..4098 over a cache prefilled to 4096
   positions, eager and graph-replayed: logits, residual and the cache rows
   the steps wrote, bit-exact with the oracle.
-- 160 prompt tokens at positions 3930..4089 in chunks of 128: the first
-  chunk ends at 4058, where the prefill's attention values run the GQA
-  kernel (the eight query heads of a kv head in one workgroup); the second
-  ends at 4090, past that kernel's LDS limit (4088 at this shape), where
-  they run per query head.  Every position's logits, the last residual and
-  the written cache rows, bit-exact with the oracle.
+- 160 prompt tokens at positions 3930..4089 in chunks of 128 and 32 tokens
+  (softmax and values as two launches).  Every position's logits, the last
+  residual and the written cache rows, bit-exact with the oracle.
 """
 import numpy as np
 import pytest
