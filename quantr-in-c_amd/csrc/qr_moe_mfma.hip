@@ -854,8 +854,12 @@ hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const ui
   }
   // items of up to 16 pairs: an expert rarely has more than one, so its rows
   // are read about once and the hint keeps the activation records cached;
-  // with 32-pair items hot experts are re-read by several items
-  a.wnt = tile <= 16;
+  // with 32-pair items hot experts are re-read by several items.  Never for the
+  // tiled layout: a 128-byte line holds a chunk of eight stages of its row, and
+  // under the hint it was gone before the next stage wanted it (Q4_K 4608 x 5632,
+  // 300 rows 174 us, 106 without; 131 rows of a matrix no cache holds 84 and 57;
+  // 4608 x 2048 28 and 25)
+  a.wnt = tile <= 16 && !tiled;
   // one expert (a dense product): with fewer than two workgroups of 64 rows per CU, workgroups of 32 rows
   // and a two-slot ring for its long rows (each workgroup walks them alone)
   int nw = 4;
