@@ -68,6 +68,7 @@ struct MF {
 // The bits of the float 1.5 * 2^23: adding an integer |S| < 2^22 to them
 // gives the bits of the float 1.5 * 2^23 + S.
 constexpr int kMagic = 0x4B400000;
+typedef float v2f __attribute__((ext_vector_type(2)));
 // The largest |bsum| whose product with any min is exact: a min is a half times
 // 0..3, at most 3 * 2047 = 6141 units of its last place, and 6141 * 2732 < 2^24.
 constexpr float kBsumExact = 2732.0f;
@@ -505,6 +506,14 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
       // of its units
       constexpr int UPL = NMAT * WR * 8 / 64 < 4 ? 2 : 4, PARTS = 8 / UPL;
       bool odd = false;  // a block scale that is not finite, or an inexact m * bsum
+      // the bsums that decide the latter, read before the scales' own round trips
+      constexpr int NBS = MF<TYPE>::kMin ? G::NTOK * 8 / 64 : 1;
+      float bsv[NBS];
+      if constexpr (MF<TYPE>::kMin) {
+#pragma unroll
+        for (int k = 0; k < NBS; k++)  // records past np repeat the first pair's
+          bsv[k] = lds_at<float>(bsA0 + (uint32_t)(slot * G::AST), k * 8 * 16 * G::APC);
+      }
       for (int i = lane; i < NMAT * WR * PARTS; i += 64) {
         const int m = i / (PARTS * WR), rem = i - m * PARTS * WR;
         const int rr = rem / PARTS, u0 = (rem - rr * PARTS) * UPL;
@@ -549,10 +558,8 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
       // scale of the wave's rows finite (checked where they were decoded) and,
       // with mins, |bsum| <= kBsumExact in every unit of the item's pairs.
       if constexpr (MF<TYPE>::kMin) {
-        const uint32_t bsA = bsA0 + ao;
 #pragma unroll
-        for (int k = 0; k < G::NTOK * 8 / 64; k++)  // records past np repeat the first pair's
-          odd |= __builtin_fabsf(lds_at<float>(bsA, k * 8 * 16 * G::APC)) > kBsumExact;
+        for (int k = 0; k < NBS; k++) odd |= __builtin_fabsf(bsv[k]) > kBsumExact;
       }
       const bool fused = __builtin_amdgcn_ballot_w64(odd) == 0;  // wave-uniform
       // One term from the accumulator bits of 1.5 * 2^23 + isum.  Fused: the
@@ -614,8 +621,14 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
               const int o = (i & 1) * (16 * G::APC) + s * kXQ;
-              bd[i] = lds_at<float>(asB[j][i >> 1], o);
-              bsf[i] = MF<TYPE>::kMin ? lds_at<float>(asB[j][i >> 1], o + 4) : 0.0f;
+              if constexpr (MF<TYPE>::kMin) {  // one read for two pairs
+                const v2f b = lds_at<v2f>(asB[j][i >> 1], o);
+                bd[i] = b.x;
+                bsf[i] = b.y;
+              } else {
+                bd[i] = lds_at<float>(asB[j][i >> 1], o);
+                bsf[i] = 0.0f;
+              }
             }
             // the accumulators start at the bits of 1.5 * 2^23, so an exact sum
             // S (|S| < 2^22) comes out as the bits of the float 1.5 * 2^23 + S;
