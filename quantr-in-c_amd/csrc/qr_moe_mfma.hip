@@ -523,7 +523,7 @@ __global__ __launch_bounds__(64 * NW) void k_expert_mfma(MfmaArgs a) {
         const int row = rw0 + rr;
         if (u0 < su && row < a.rows) {
           const uint32_t hd = ALN ? 0u : ((uint32_t)row * (uint32_t)rb + s0) & 15u;
-          odd = unit_scales<TYPE, UPL>(
+          odd |= unit_scales<TYPE, UPL>(
               wl0 + (uint32_t)(slot * G::WST + (m * WR + rr) * G::SLOT) + hd, u0, su, sc, mn);
         }
 #pragma unroll
