@@ -478,29 +478,60 @@ static hipError_t launch_blk_k(const GemvArgs& a, int grid, size_t lds, hipStrea
 }
 
 // How many of a call's nt tokens share a workgroup; the rest are further rows
-// of workgroups (grid y) in the same launch, whose reads of the matrix the
-// caches serve.  Sharing saves decoding and LDS traffic, but it multiplies a
-// wave's serial work, so it pays only where the tiles fill the chip by
-// themselves: up to four tiles per CU (one per SIMD) the tokens go apart, by
-// twos where a token's tile work is long (Q5_K, Q6_K).  Measured, together and as
-// chosen, us: 5632 x 2048, four tokens, Q4_K tiled 7.8 -> 5.2 and row-major
-// 8.0 -> 5.6, Q5_K 8.2 -> 6.9, Q6_K 8.7 -> 8.0, Q8_0 7.7 -> 7.1 (three tokens
-// of Q6_K / Q8_0 apart: 7.3 -> 9.3, 6.6 -> 8.0, so they stay together); 2048 x
-// 5632, four tokens, 13.8 -> 9.9, 13.4 -> 10.6, 14.4 -> 11.6, 13.1 -> 9.6.  With
-// more tiles only Q4_K gains, in twos (32000 x 2048, four tokens: 14.1 -> 12.1;
-// Q5_K 16.3 -> 17.6, Q6_K 18.0 -> 21.3, Q8_0 18.3 -> 20.1, not taken).  Eight
-// tokens are one launch instead of two of four: 32000 x 2048 28.0 -> 19.4,
-// 32.5 -> 25.4, 36.0 -> 28.6, 36.5 -> 27.6.
-static int tokens_per_row(int type, bool tiled_k, int nt, int ntiles) {
-  const bool heavy = type == QR_T_Q5_K || type == QR_T_Q6_K;
-  const bool few = ntiles <= 4 * device_cus();
-  switch (nt) {
-    case 2: return few ? 1 : 2;
-    case 3: return few && (type == QR_T_Q4_K || (type == QR_T_Q5_K && tiled_k)) ? 1 : 3;
-    case 4: return few ? (heavy ? 2 : 1) : type == QR_T_Q4_K ? 2 : 4;
-    case 8: return few ? (heavy ? 2 : 1) : heavy ? 4 : 2;
-    default: return nt == 1 ? 1 : 0;  // 0: not a width of these kernels
+// of workgroups (grid y) in the same launch.  Sharing decodes a weight once and
+// reads the matrix once; apart, each group of tokens has a shorter start-up (its
+// quantization), less serial work per wave and more waves, and re-reads the matrix
+// through the caches.  So it is a matter of the (tile, token group)s per CU: apart
+// up to a line a + b nb (nb: super-blocks of a row; longer rows start up longer), in
+// twos up to a second one, together (eight as two rows of four) beyond.  The lines
+// are fitted over rows of 256 to 32000 by 512 to 5632, with the matrix in the
+// caches and from memory, so that no choice is slower than together by more than
+// the runs differ.
+// Where they lie differs by how dear the decoding is (Q4_K cheapest) and by the
+// workgroups that the tokens' activations leave room for (long rows).  us together,
+// apart, in twos, the matrix in the caches: Q4_K tiled 2048 x 5632, four tokens 13.7 /
+// 10.3 / 10.7; 5632 x 5632, four 19.0 / 16.5 / 24.2; 32000 x 2048, four 14.6 / 14.8 /
+// 12.5; row-major 5632 x 2048, four, Q4_K 8.2 / 5.9 / 6.8, Q5_K 8.3 / 8.7 / 7.5; Q6_K
+// tiled 5632 x 2048, four 8.8 / 9.8 / 8.1; Q6_K tiled 32000 x 512, two 5.9 / 6.6 (from
+// memory 6.9 / 8.2); Q8_0 tiled 16000 x 5632, eight 77.5 / 82.7 / 98.5.
+struct SplitLine {
+  float a, b;
+};
+struct TokenSplit {
+  SplitLine one[4];  // 2, 3, 4 and 8 tokens: each apart
+  SplitLine two[2];  // 4 and 8 tokens: in twos ...
+  int two_nb;        // ... for rows of at most so many super-blocks
+};
+constexpr TokenSplit kSplitRowsQ4 = {{{-2, 2}, {2, 3}, {-2, 4}, {-4, 4}}, {{48, 0.25f}, {6, 6}}, 64};
+constexpr TokenSplit kSplitRowsQ5 = {{{3, 0.25f}, {4, 0.5f}, {2, 0.5f}, {4, 0}}, {{4, 0.75f}, {-4, 4}}, 64};
+constexpr TokenSplit kSplitTiledQ4 = {{{-2, 2}, {5, 4}, {1, 2.5f}, {4, 4}}, {{24, 1}, {-24, 11}}, 17};
+constexpr TokenSplit kSplitTiledQ5 = {{{3, 0.5f}, {5, 0.5f}, {4, 0.5f}, {2, 0.5f}}, {{4, 0.75f}, {6, 2}}, 64};
+constexpr TokenSplit kSplitTiledQ6 = {{{3, 0.25f}, {2, 0.5f}, {3, 0.25f}, {4, 0}}, {{2, 1}, {2, 1}}, 64};
+constexpr TokenSplit kSplitTiledQ8 = {{{2, 0.5f}, {3, 0.5f}, {0, 2}, {-2, 3}}, {{4, 0.75f}, {64, 0.25f}}, 12};
+
+static int tokens_per_row(const TokenSplit& s, int nt, int nb, int ntiles) {
+  if (nt == 1) return 1;
+  const int i = nt == 2 ? 0 : nt == 3 ? 1 : nt == 4 ? 2 : nt == 8 ? 3 : -1;
+  if (i < 0) return 0;  // not a width of these kernels
+  const auto within = [&](int m, SplitLine l) {
+    return (float)ntiles * (float)(nt / m) <= (l.a + l.b * (float)nb) * (float)device_cus();
+  };
+  if (within(1, s.one[i])) return 1;
+  if (i >= 2 && nb <= s.two_nb && within(2, s.two[i - 2])) return 2;
+  return nt == 8 ? 4 : nt;
+}
+
+// Workgroups of one token row: those that want tiles, at most cap.  With several
+// rows a multiple of eight, so that the rows' workgroups of the same tiles are on
+// the same XCD (workgroups go to the eight in turn) and read the matrix from its
+// L2 once: from memory, 16000 x 512 Q4_K tiled, eight tokens apart 8.1 -> 5.9 us, Q8_0
+// tiled, four apart 8.4 -> 6.5.  A workgroup past the last tile does nothing.
+static int row_grid(int want, int cap, int rows) {
+  if (rows > 1 && cap >= 8) {
+    want = (want + 7) & ~7;
+    cap &= ~7;
   }
+  return want < cap ? want : cap;
 }
 
 // One tile in flight per wave and as many workgroups per CU as LDS holds, up
@@ -521,8 +552,7 @@ static hipError_t launch_blk_t(const GemvArgs& a, hipStream_t st, int ny = 1) {
   const int want = (ntiles + kBlkWaves - 1) / kBlkWaves;
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 3 ? 3 : per_cu);
-  const int cap = std::max(1, device_cus() * per_cu / ny);
-  const int grid = want < cap ? want : cap;
+  const int grid = row_grid(want, std::max(1, device_cus() * per_cu / ny), ny);
   if (grid <= 0) return hipSuccess;
   const bool acc = a.acc || a.accb;
   if (xs) return acc ? launch_blk_k<TYPE, NT, true, true>(a, grid, lds, st, ny)
@@ -590,7 +620,8 @@ static hipError_t launch_nt(const GemvArgs& a, int nt, hipStream_t st) {
     // (the parity mode's integer sums: NT tokens per workgroup, below)
     if (nt > 1 && !a.acc && !a.accb && gemv_blk_ok(TYPE, a.d, nt == 8 ? 4 : nt)) {
       const int RB = 64 / (a.d >> 8);
-      const int m = tokens_per_row(TYPE, false, nt, (a.n + RB - 1) / RB);
+      const int m = tokens_per_row(TYPE == QR_T_Q4_K ? kSplitRowsQ4 : kSplitRowsQ5, nt, a.d >> 8,
+                                   (a.n + RB - 1) / RB);
       switch (m) {
         case 1: return launch_blk_t<TYPE, 1>(a, st, nt);
         case 2: return launch_blk_t<TYPE, 2>(a, st, nt / 2);
@@ -651,8 +682,7 @@ static hipError_t launch_sq_nw(const GemvArgs& a, hipStream_t st, int ny) {
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
   const int want = (g.ntiles + NW - 1) / NW;
-  const int cap = std::max(1, device_cus() * per_cu / ny);
-  const int grid = want < cap ? want : cap;
+  const int grid = row_grid(want, std::max(1, device_cus() * per_cu / ny), ny);
   hipLaunchKernelGGL((k_gemv_tiled_sq<TYPE, NT, NW>), dim3(grid, ny), dim3(64 * NW), lds, st, a);
   return hipGetLastError();
 }
@@ -664,7 +694,8 @@ static hipError_t launch_sq_t(const GemvArgs& a, hipStream_t st, int ny = 1) {
 
 template <int TYPE>
 static hipError_t launch_sq_type(const GemvArgs& a, int nt, hipStream_t st) {
-  const int m = tokens_per_row(TYPE, false, nt, a.t_ntiles);
+  const int m = tokens_per_row(TYPE == QR_T_Q6_K ? kSplitTiledQ6 : kSplitTiledQ8, nt, a.t_nb,
+                               a.t_ntiles);
   switch (m) {
     case 1: return launch_sq_t<TYPE, 1>(a, st, nt);
     case 2: return launch_sq_t<TYPE, 2>(a, st, nt / 2);
@@ -713,15 +744,15 @@ static hipError_t launch_tiled_t(const GemvArgs& a, hipStream_t st, int ny = 1) 
   int per_cu = (int)(kLdsMax / lds);
   per_cu = per_cu < 1 ? 1 : (per_cu > 4 ? 4 : per_cu);
   const int want = (g.ntiles + nw - 1) / nw;
-  const int cap = std::max(1, cus * per_cu / ny);
-  const int grid = want < cap ? want : cap;
+  const int grid = row_grid(want, std::max(1, cus * per_cu / ny), ny);
   if (nw == 8) return launch_tiled_nw<TYPE, NT, 8>(a, grid, lds, st, ny);
   return launch_tiled_nw<TYPE, NT, 4>(a, grid, lds, st, ny);
 }
 
 template <int TYPE>
 static hipError_t launch_tiled_type(const GemvArgs& a, int nt, hipStream_t st) {
-  const int m = tokens_per_row(TYPE, true, nt, a.t_ntiles);
+  const int m = tokens_per_row(TYPE == QR_T_Q4_K ? kSplitTiledQ4 : kSplitTiledQ5, nt, a.t_nb,
+                               a.t_ntiles);
   switch (m) {
     case 1: return launch_tiled_t<TYPE, 1>(a, st, nt);
     case 2: return launch_tiled_t<TYPE, 2>(a, st, nt / 2);
