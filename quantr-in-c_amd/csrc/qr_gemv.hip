@@ -508,6 +508,9 @@ constexpr TokenSplit kSplitTiledQ4 = {{{-2, 2}, {5, 4}, {1, 2.5f}, {4, 4}}, {{24
 constexpr TokenSplit kSplitTiledQ5 = {{{3, 0.5f}, {5, 0.5f}, {4, 0.5f}, {2, 0.5f}}, {{4, 0.75f}, {6, 2}}, 64};
 constexpr TokenSplit kSplitTiledQ6 = {{{3, 0.25f}, {2, 0.5f}, {3, 0.25f}, {4, 0}}, {{2, 1}, {2, 1}}, 64};
 constexpr TokenSplit kSplitTiledQ8 = {{{2, 0.5f}, {3, 0.5f}, {0, 2}, {-2, 3}}, {{4, 0.75f}, {64, 0.25f}}, 12};
+constexpr TokenSplit kSplitGgmlQ4 = {{{1e6f, 0}, {1e6f, 0}, {1e6f, 0}, {48, 6}}, {{0, 0}, {-24, 16}}, 64};
+constexpr TokenSplit kSplitGgmlQ5 = {{{12, 4}, {-4, 8}, {4, 8}, {12, 8}}, {{12, 4}, {12, 4}}, 64};
+constexpr TokenSplit kSplitGgmlQ6 = {{{2, 1.5f}, {2, 2}, {-4, 4}, {-4, 4}}, {{-4, 4}, {-4, 4}}, 64};
 
 static int tokens_per_row(const TokenSplit& s, int nt, int nb, int ntiles) {
   if (nt == 1) return 1;
@@ -978,6 +981,7 @@ static hipError_t launch_ggml_x(const GemvArgs& a, hipStream_t st, int pairs = 0
   int grid = (want + rounds - 1) / rounds;
   if (grid < 1) grid = 1;
   if (ntiles <= 0) return hipSuccess;
+  if (pairs > 1 && !a.eidx) grid = (grid + 7) & ~7;  // token rows: see row_grid
   hipLaunchKernelGGL((k_gemv_ggml<T, NT, XM, G>), dim3(grid, pairs > 0 ? pairs : 1), dim3(256),
                      lds, st, a);
   return hipGetLastError();
@@ -994,31 +998,25 @@ static hipError_t launch_ggml_t(const GemvArgs& a, hipStream_t st, int pairs = 0
                           : launch_ggml_x<T, NT, kXmLate>(a, st, pairs);
 }
 
-// Several tokens: each token its own row of workgroups (grid y), or several
-// per workgroup, sharing the decoding of the weights.  A lane computes a whole
-// super-block, so one token's pass leaves a wave a long serial piece that more
-// tokens per wave only lengthen, while the matrix's second reader finds it in
-// the caches.  Single tokens wherever one token's tiles are at most three
-// workgroups per CU (Q4_K / Q5_K / Q6_K: 5632 x 2048, three tokens, 14.6 / 14.3 /
-// 17.1 us together, 6.8 / 7.6 / 15.6 apart; 2048 x 5632, eight, 74 / 75 / 82
-// against 24 / 26 / 34; 12000 x 3072, four, 33 / 35 / 44 against 19 / 24 / 35).
-// Beyond that only Q4_K's cheap decoding stands the repetition (32000 x 2048,
-// four tokens: 27.2 together, 25.6 apart; Q5_K 28.8 and 32.2, Q6_K 38.3 and
-// 49.3), and eight tokens are two rows of four in one launch (32000 x 2048:
-// 41.4 / 44.2 / 63.9 us; apart 48.9 / 59.2 / 88.1; one after the other
-// 54.3 / 57.7 / 76.6).
+// Several tokens (tokens_per_row): a lane computes a whole super-block, so one
+// token's pass leaves a wave a long serial piece that more tokens per wave only
+// lengthen, and tokens go apart far longer than in the kernels above.  us together,
+// apart, in twos, the matrix in the caches: 5632 x 2048, four tokens, Q4_K 17.3 / 7.2 /
+// 12.4, Q6_K 21.1 / 16.6 / 16.5; 32000 x 512, three tokens, Q6_K 11.6 / 13.8; eight
+// tokens, 32000 x 2048, Q4_K 40.8 / 39.9 / 43.9, Q5_K 43.9 / 49.1 / 50.1, 24000 x 2048, Q6_K
+// 50.9 / 65.6 / 57.7.  Weights that no cache holds (copies in turn) say the same:
+// 5632 x 2048, four tokens, Q4_K 18.3 / 7.8 / 13.1, Q6_K 22.2 / 17.7 / 17.4.
 template <int T>
-static hipError_t launch_ggml_type(GemvArgs a, int nt, hipStream_t st) {
-  const int RB = 64 / (a.d >> 8);
-  const int want = ((a.n + RB - 1) / RB + 3) / 4;
-  const bool apart = want <= 3 * device_cus() || (T == kGgmlQ4 && nt <= 4);
-  if (nt > 1 && apart) return launch_ggml_t<T, 1>(a, st, nt);
-  switch (nt) {
-    case 1: return launch_ggml_t<T, 1>(a, st);
-    case 2: return launch_ggml_t<T, 2>(a, st);
-    case 3: return launch_ggml_t<T, 3>(a, st);
-    case 4: return launch_ggml_t<T, 4>(a, st);
-    case 8: return launch_ggml_t<T, 4>(a, st, 2);
+static hipError_t launch_ggml_type(const GemvArgs& a, int nt, hipStream_t st) {
+  const int nb = a.d >> 8, RB = 64 / nb;
+  const int m = tokens_per_row(T == kGgmlQ4 ? kSplitGgmlQ4 : T == kGgmlQ5 ? kSplitGgmlQ5 : kSplitGgmlQ6,
+                               nt, nb, (a.n + RB - 1) / RB);
+  const int rows = m > 0 && nt > m ? nt / m : 0;
+  switch (m) {
+    case 1: return launch_ggml_t<T, 1>(a, st, rows);
+    case 2: return launch_ggml_t<T, 2>(a, st, rows);
+    case 3: return launch_ggml_t<T, 3>(a, st, rows);
+    case 4: return launch_ggml_t<T, 4>(a, st, rows);
     default: return hipErrorInvalidValue;
   }
 }

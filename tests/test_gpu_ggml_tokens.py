@@ -1,5 +1,5 @@
 """The llama.cpp-layout GEMV of several tokens on both sides of its split: each
-token its own row of workgroups (few tiles), or several tokens per workgroup
+token its own row of workgroups (few tiles), two, or several tokens per workgroup
 and two rows of four (many tiles), with strided tokens and outputs.  Bit-exact
 with the oracle.
 """
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("nt", [2, 3, 4, 8])
-@pytest.mark.parametrize("n,d", [(65, 768), (24601, 2048)])
+@pytest.mark.parametrize("n,d", [(65, 768), (24601, 2048), (50001, 512)])
 @pytest.mark.parametrize("qtype", [GB.Q4_K, GB.Q5_K, GB.Q6_K])
 def test_ggml_tokens(dev, oracle, qtype, n, d, nt):
     W = GB.random_rows(90 + qtype, qtype, n, d)
