@@ -590,18 +590,42 @@ static hipError_t launch_mt_t(const GemvArgs& a, hipStream_t st, int quads = 1) 
   return hipGetLastError();
 }
 
+// Calls that the kernels below serve faster than the MFMA kernel.
+// - Few long rows (n no more than the CUs, so a tile of 16 rows for every
+//   16th): a tile's stages are one chain, the general kernel has a workgroup per
+//   row.  Two tokens, 256 x 5632, Q8_0 in the AVX-512 order 16.7 us there and 19.6
+//   here, 256 x 2080 9.8 and 10.6, three tokens 256 x 5632 19.0 and 21.0; Q6_K two
+//   tokens 256 x 5632 10.4 and 11.1.  (AVX2 order, two tokens: 20.7 and 15.4.)
+// - Two tokens of many short Q6_K rows that don't stream: the stages of a tile do not
+//   divide among the eight waves.  16000 x 768 7.4 us (from memory 8.4) and 8.9 (9.1),
+//   8192 x 768 5.3 (6.3) and 6.9 (6.9).
+// (Two tokens of 16000 x 512 in the AVX-512 order, 8.3 us here and 7.1 streamed with
+// the matrix in the caches, are level from memory: 8.7 each.)
+static bool mt_slower(int type, int q8o, int nt, int n, int U) {
+  const bool avx512 = type == QR_T_Q8_0 && q8o == kQ8Avx512;
+  if ((avx512 || type == QR_T_Q6_K) && n <= device_cus() && U > (avx512 ? 64 : 160) * (nt - 1))
+    return true;
+  return type == QR_T_Q6_K && nt == 2 && U < 48 && 64 % U != 0 &&
+         (n + kMtRows - 1) / kMtRows >= 2 * device_cus();
+}
+
 template <int TYPE, int NT, int Q8O>
 static hipError_t launch_any_t(const GemvArgs& a, hipStream_t st) {
   if constexpr ((TYPE == QR_T_Q4_K || TYPE == QR_T_Q5_K) && NT <= 4) {
     if (gemv_blk_ok(TYPE, a.d, NT)) return launch_blk_t<TYPE, NT>(a, st);
   }
-  // Q6_K / Q8_0 of several tokens: the MFMA kernel (figures in qr_gemv_mt.h).
-  // Two tokens of Q8_0 in the sequential order stay with the kernels below: the
-  // streaming engine takes 20.1 us on 32000 x 2048 where this one takes 22.0.
-  // The integer sums of the parity mode are formed by the kernels below only.
+  // Q6_K / Q8_0 of several tokens: the MFMA kernel (figures in qr_gemv_mt.h), except
+  // where mt_slower says and for two tokens of Q8_0 in the sequential order.  Where
+  // these stream (rows of 16, 32 or 64 blocks) the two are close (32000 x 2048 20.5
+  // us streamed, 21.9 here; 16000 x 2048 15.6 and 14.1); the others go to the
+  // general kernel, which is ahead for short rows (8192 x 1536 7.1 us, here 8.7) and
+  // behind for long ones (8192 x 5632 32.9 and 18.7): no line is drawn between
+  // them.  The integer sums of the parity mode are formed by the kernels below
+  // only.
   constexpr bool kSeqQ8 = TYPE == QR_T_Q8_0 && Q8O == kQ8Seq;
   if constexpr ((TYPE == QR_T_Q6_K || TYPE == QR_T_Q8_0) && (NT > 2 || (NT == 2 && !kSeqQ8))) {
-    if (!a.acc && !a.accb && qr_units(TYPE, a.d) > 0) {
+    if (!a.acc && !a.accb && qr_units(TYPE, a.d) > 0 &&
+        !mt_slower(TYPE, Q8O, NT, a.n, qr_units(TYPE, a.d))) {
       if constexpr (q8_slots(TYPE, Q8O) == 9 && NT == 8) {
         if (mt_lds_bytes<TYPE, 4, Q8O>(qr_units(TYPE, a.d)) <= kLdsMax)
           return launch_mt_t<TYPE, 4, Q8O>(a, st, 2);

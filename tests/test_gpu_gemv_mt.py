@@ -14,8 +14,10 @@ from quantr_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-Q8_SHAPES = [(1, 32), (15, 64), (16, 256), (17, 288), (33, 608), (83, 2144), (4100, 96)]
-K_SHAPES = [(1, 256), (17, 512), (333, 768), (40, 1792), (4099, 2304)]
+Q8_SHAPES = [(1, 32), (15, 64), (16, 256), (17, 288), (33, 608), (83, 2144), (4100, 96),
+             (256, 2144), (257, 2144)]  # the last two: a line of the route (as many rows as CUs)
+K_SHAPES = [(1, 256), (17, 512), (333, 768), (40, 1792), (4099, 2304),
+            (8176, 768), (8177, 768), (256, 5632), (257, 5632)]  # lines of the route
 CASES = ([(Q.TYPE_Q8_0, o, n, d) for o in (ORDER_SEQ, ORDER_AVX2, ORDER_AVX512) for n, d in Q8_SHAPES]
          + [(Q.TYPE_Q6_K, ORDER_SEQ, n, d) for n, d in K_SHAPES]
          + [(t, ORDER_SEQ, n, d) for t in (Q.TYPE_Q4_K, Q.TYPE_Q5_K) for n, d in K_SHAPES[:3]])
