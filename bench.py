@@ -58,10 +58,12 @@ HBM_PEAK_GBPS = 8000.0
 # fp32 VALU lane operations per second without packed instructions: 256 CUs x 4 SIMDs x 16
 # lanes x 2.4 GHz (the published 157.3 TFLOP/s counts packed FMAs as 4 flops per lane)
 VALU_PEAK_OPS = 256 * 64 * 2.4e9
-# fp32 operations per (output row, token, 32-element unit) that the reference's dot rounds
-# one by one: (sc * isum - m * bsum) * bd added on (Q4_K / Q5_K), sc * isum * bd added on
-# (Q6_K), isum * (da * db) added on (Q8_0), each after the int -> float conversion
-TERM_OPS = {Q.TYPE_Q4_K: 6, Q.TYPE_Q5_K: 6, Q.TYPE_Q6_K: 4, Q.TYPE_Q8_0: 4}
+# fp32 operations per (output row, token, 32-element unit) that give the reference's dot,
+# (sc * isum - m * bsum) * bd added on (Q4_K / Q5_K) or sc * isum * bd added on (Q6_K,
+# Q8_0), with its roundings: one multiply-add from the integer sum's float bits (its product
+# and the conversion are exact together), one more for the exact m * bsum, the multiply by
+# bd and the add
+TERM_OPS = {Q.TYPE_Q4_K: 4, Q.TYPE_Q5_K: 4, Q.TYPE_Q6_K: 3, Q.TYPE_Q8_0: 3}
 METRIC = "Q4_K GEMV weight GB/s (% HBM peak); MoE layer tokens/s at 30B-A3B shape"
 TNAME = {Q.TYPE_Q8_0: "Q8_0", Q.TYPE_Q4_K: "Q4_K", Q.TYPE_Q5_K: "Q5_K", Q.TYPE_Q6_K: "Q6_K"}
 TINYLLAMA = [(2048, 2048), (256, 2048), (5632, 2048), (2048, 5632)]

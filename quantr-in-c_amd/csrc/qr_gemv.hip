@@ -355,8 +355,10 @@ bool gemv_stream_ok(int type, int q8o, int d, int nt) {
 // Workgroups per CU of the streaming kernel: 3 for one or two tokens, 2 for
 // more, fewer where LDS does not hold that many.  Measured on 32000 x 2048
 // Q6_K / Q8_0 and the 151936 x 2048 Q6_K lm_head: 3 per CU streams 4.3 TB/s
-// for one token where 2 and 4 give 3.6-4.0 and 1 gives 2.6; with 4 tokens 2
-// per CU takes 28.9 us where 3 takes 33.8 (Q6_K) and 40.8 (Q8_0).
+// for one token where 2 and 4 give 3.6-4.0 and 1 gives 2.6.  Several tokens come
+// here only for the parity mode's integer sums, where the MFMA kernel's LDS does not
+// hold them or mt_slower sends them, and two of Q8_0 in the sequential order; with
+// 4, 2 per CU took 28.9 us where 3 took 33.8 (Q6_K) and 40.8 (Q8_0).
 template <int TYPE, int NT, int Q8O>
 static hipError_t launch_stream_t(const GemvArgs& a, hipStream_t st) {
   const TileShape sh = tile_shape(TYPE, a.d, Q8O);

@@ -15,8 +15,9 @@
 // unit order, so every output equals the reference's sequential fused dot.
 // Two fused multiply-adds stand for four of its operations where both their
 // inner products are exact (term_of below): the T = 512 layer of the
-// Qwen3-30B-A3B shape 242.9 -> 228.3 us, with 48 M VALU instructions in the
-// gate/up product where it had 58 M, and 40 M in down where it had 47 M.
+// Qwen3-30B-A3B shape 242.9 -> 228.3 us.  The products there issue 45 M and 31 M
+// VALU instructions (58 M and 47 M once), 62 % and 65 % of their time, of which the
+// terms need 25 M and 9.4 M: operands, scales, DMA and set-up take the rest.
 //
 // MFMA lane layout (v_mfma_i32_16x16x32_i8, checked on the device): A, the
 // pairs, is lane -> pair lane%16, elements 8*(lane/16)..+7 of the unit; B, the
@@ -873,8 +874,9 @@ hipError_t expert_mfma_launch(int type, bool gateup, const uint8_t* W1, const ui
   // 300 rows 174 us, 106 without; 131 rows of a matrix no cache holds 84 and 57;
   // 4608 x 2048 28 and 25)
   a.wnt = tile <= 16 && !tiled;
-  // one expert (a dense product): with fewer than two workgroups of 64 rows per CU, workgroups of 32 rows
-  // and a two-slot ring for its long rows (each workgroup walks them alone)
+  // one expert (a dense product): with fewer than two workgroups of 64 rows per
+  // CU, workgroups of 32 rows; a two-slot ring for its long rows (each workgroup
+  // walks them alone)
   int nw = 4;
   if (E == 1 && (long)((rows + 63) / 64) * ((P + tile - 1) / tile) < 2L * device_cus()) nw = 2;
   const int stages = type == QR_T_Q8_0 ? (cols / 32 + 7) / 8 : cols / 256;

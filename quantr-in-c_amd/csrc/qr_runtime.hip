@@ -589,6 +589,9 @@ int qr_gemv_ord(qr_ctx* c, int order, uint32_t type, const void* w, const float*
            "k_gemv_tiled");
     return QR_OK;
   }
+  // Several tokens are admitted by the LDS of the block, streaming and general
+  // kernels, whichever kernel then takes them: eight by the general one's, so longer
+  // rows of eight are refused although the kernels that serve eight would hold them.
   const int R = qr::gemv_rows_per_wg((int)type, order, n, d, nt);
   if (!qr::gemv_blk_ok((int)type, d, nt) && !qr::gemv_stream_ok((int)type, order, d, nt) &&
       qr::gemv_lds_bytes((int)type, order, d, nt, R) > 64 * 1024)

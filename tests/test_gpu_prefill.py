@@ -155,10 +155,10 @@ def test_prefill_head128_chunks(dev, oracle, source, page):
 @pytest.mark.parametrize("kv_type,page", [(Q.KV_Q8_0, 64), (Q.KV_F32, 16), (Q.KV_F16, 32)],
                          ids=["q8_0_pages64", "f32_pages16", "f16_pages32"])
 def test_prefill_gqa8_chunks(dev, oracle, kv_type, page):
-    """GQA 8:1 at head_dim 128, the shape whose prefill attention values run
-    the query heads of a kv head in one workgroup (V staged once for the
-    eight): 300 prompt tokens in chunks of 128 against the oracle, every
-    token's logits, the last residual and the cache rows bit for bit."""
+    """GQA 8:1 at head_dim 128: 300 prompt tokens in chunks of 128, 128 and 44
+    (Q8_0 and fp16: V staged once for several query heads of the kv head, then per
+    head; fp32 per head) against the oracle, every token's logits, the last
+    residual and the cache rows bit for bit."""
     m = I.qwen3_small_model(n_layers=2, seq_len=320, n_kv_heads=1)
     rng = np.random.default_rng(19)
     toks = rng.integers(0, m["vocab"], size=300).astype(np.int32)
