@@ -603,12 +603,18 @@ static hipError_t launch_mt_t(const GemvArgs& a, hipStream_t st, int quads = 1) 
 //   8192 x 768 5.3 (6.3) and 6.9 (6.9).
 // (Two tokens of 16000 x 512 in the AVX-512 order, 8.3 us here and 7.1 streamed with
 // the matrix in the caches, are level from memory: 8.7 each.)
-static bool mt_slower(int type, int q8o, int nt, int n, int U) {
+static bool mt_slower(int type, int q8o, int nt, const GemvArgs& a) {
+  if (nt > 3) return false;
+  const int U = qr_units(type, a.d);
   const bool avx512 = type == QR_T_Q8_0 && q8o == kQ8Avx512;
-  if ((avx512 || type == QR_T_Q6_K) && n <= device_cus() && U > (avx512 ? 64 : 160) * (nt - 1))
-    return true;
-  return type == QR_T_Q6_K && nt == 2 && U < 48 && 64 % U != 0 &&
-         (n + kMtRows - 1) / kMtRows >= 2 * device_cus();
+  const bool few_long = (avx512 || type == QR_T_Q6_K) && a.n <= device_cus() &&
+                        U > (avx512 ? 64 : 160) * (nt - 1);
+  const bool many_short = type == QR_T_Q6_K && nt == 2 && U < 48 && 64 % U != 0 &&
+                          (a.n + kMtRows - 1) / kMtRows >= 2 * device_cus();
+  // (rows that neither of those kernels holds stay)
+  return (few_long || many_short) &&
+         (gemv_stream_ok(type, q8o, a.d, nt) ||
+          gemv_lds_bytes(type, q8o, a.d, nt, a.rows_per_wg) <= 64 * 1024);
 }
 
 template <int TYPE, int NT, int Q8O>
@@ -627,7 +633,7 @@ static hipError_t launch_any_t(const GemvArgs& a, hipStream_t st) {
   constexpr bool kSeqQ8 = TYPE == QR_T_Q8_0 && Q8O == kQ8Seq;
   if constexpr ((TYPE == QR_T_Q6_K || TYPE == QR_T_Q8_0) && (NT > 2 || (NT == 2 && !kSeqQ8))) {
     if (!a.acc && !a.accb && qr_units(TYPE, a.d) > 0 &&
-        !mt_slower(TYPE, Q8O, NT, a.n, qr_units(TYPE, a.d))) {
+        !mt_slower(TYPE, Q8O, NT, a)) {
       if constexpr (q8_slots(TYPE, Q8O) == 9 && NT == 8) {
         if (mt_lds_bytes<TYPE, 4, Q8O>(qr_units(TYPE, a.d)) <= kLdsMax)
           return launch_mt_t<TYPE, 4, Q8O>(a, st, 2);

@@ -11,7 +11,7 @@ import pytest
 import inputs as I
 import quantr_amd as Q
 from conftest import assert_bits_equal
-from oracle import ORDER_AVX2
+from oracle import ORDER_AVX2, ORDER_AVX512
 from test_gpu_prefill import make_decoder, prefill
 
 pytestmark = pytest.mark.gpu
@@ -90,3 +90,35 @@ def test_prefill_extent_lines(dev, oracle, extent, kv_type):
     workgroup change (4096, 8192), or the two launches end (16384)."""
     m = _model(8, 1, 64, extent + 16)
     _run(dev, oracle, m, kv_type, 256, extent - 3, (3, 1, 2))
+
+
+def test_prefill_wide_lane_order_rows(dev, oracle):
+    """A k projection of as many rows as CUs, 8192 wide, Q8_0 in the AVX-512 order:
+    three tokens of it are more than the general GEMV's LDS holds."""
+    m = I.qwen3_small_model(n_layers=1, seq_len=16)
+    dim, H, hd, E, hidden = 8192, 2, 128, 2, 256
+    m.update(dim=dim, n_heads=H, n_kv_heads=H, head_dim=hd, E=E, K=1, hidden=hidden)
+    wt = m["wtype"]
+    m["tok_embd"] = I._rows(9701, m["tok_type"], m["vocab"], dim)
+    m["wcls"] = I._rows(9702, m["wcls_type"], m["vocab"], dim)
+    m["rms_final"] = (1.0 + I.activations(9703, 1, dim, std=0.1)[0]).astype(np.float32)
+    m["layers"] = [dict(
+        rms_att=(1.0 + I.activations(9704, 1, dim, std=0.1)[0]).astype(np.float32),
+        rms_ffn=(1.0 + I.activations(9705, 1, dim, std=0.1)[0]).astype(np.float32),
+        wq=I._rows(9706, wt[0], H * hd, dim), wk=I._rows(9707, wt[1], H * hd, dim),
+        wv=I._rows(9708, wt[2], H * hd, dim), wo=I._rows(9709, wt[3], dim, H * hd),
+        router=I.activations(9710, E, dim, std=0.05),
+        up=I.blocks(9711, m["up_type"], E * hidden * (dim // 256)),
+        gate=I.blocks(9712, m["up_type"], E * hidden * (dim // 256)),
+        down=I.blocks(9713, m["down_type"], E * dim * (hidden // 256)))]
+    toks = np.array([3, 7, 11], np.int32)
+    print("prefill routes wide rows", flush=True)
+    d = make_decoder(dev, m, Q.KV_F32, ORDER_AVX512, page=16)
+    lg, x = prefill(dev, d, m, toks)
+    d.close()
+    kvb = oracle.kv_row_bytes(Q.KV_F32, H * hd)
+    kc, vc = np.zeros((2, m["seq_len"], kvb), np.uint8)
+    want, xs = oracle.forward_cached(m, kc.reshape(-1), vc.reshape(-1), [int(t) for t in toks], 0,
+                                     ORDER_AVX512, Q.KV_F32)
+    assert_bits_equal(lg, want, "prefill logits")
+    assert_bits_equal(x, xs[-1], "prefill residual")
