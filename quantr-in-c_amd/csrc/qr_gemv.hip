@@ -604,7 +604,7 @@ static hipError_t launch_mt_t(const GemvArgs& a, hipStream_t st, int quads = 1) 
 // (Two tokens of 16000 x 512 in the AVX-512 order, 8.3 us here and 7.1 streamed with
 // the matrix in the caches, are level from memory: 8.7 each.)
 static bool mt_slower(int type, int q8o, int nt, const GemvArgs& a) {
-  if (nt > 3) return false;
+  if (nt > 3) return false;  // rows as long as the lines below ask for don't fit there
   const int U = qr_units(type, a.d);
   const bool avx512 = type == QR_T_Q8_0 && q8o == kQ8Avx512;
   const bool few_long = (avx512 || type == QR_T_Q6_K) && a.n <= device_cus() &&
